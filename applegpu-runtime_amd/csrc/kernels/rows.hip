@@ -11,7 +11,8 @@
 //               y = gamma*(x-mean)*inv_std + beta              :1075-1116
 // The reference runs one thread per row; here one 64-lane wavefront owns a
 // row (rows up to 2048 columns stay in registers: a single HBM read and a
-// single write), and a 256-thread workgroup owns longer rows.
+// single write); longer or unaligned rows of softmax and layer_norm are in
+// rows_reg.hip.
 #include "device.hpp"
 #include "gemm_kernels.hpp"  // x3_store4: packed x3 rows of the layer_norm output
 
@@ -217,7 +218,8 @@ __device__ __forceinline__ float block_max(float v, float* sh) {
   return fmaxf(fmaxf(sh[0], sh[1]), fmaxf(sh[2], sh[3]));
 }
 
-// ── softmax family, long rows: one 256-thread block per row, online max/sum ─
+// ── softmax family, rows past rows_reg.hip's reach: one 256-thread block per
+// row, online max/sum ─────────────────────────────────────────────────────
 template <typename T>
 __global__ void __launch_bounds__(256) softmax_block(int op, const T* __restrict__ x, int64_t ldx,
                                                      T* __restrict__ y, int64_t ldy, int64_t cols,
@@ -972,65 +974,68 @@ bool vec_ok(const void* p, int64_t ld, size_t esz) {
 
 unsigned rows_grid(int64_t rows) { return (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock); }
 
-template <typename T, int NV>
-void sm_nv(int op, const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, int64_t cols, int64_t crow,
-           bool vec, hipStream_t s) {
-  if (vec && cols == NV * 256)
-    hipLaunchKernelGGL((softmax_wave<T, NV, true>), dim3(rows_grid(rows)), dim3(256), 0, s, op, (const T*)x, ldx,
-                       (T*)y, ldy, rows, cols, crow, vec);
-  else
-    hipLaunchKernelGGL((softmax_wave<T, NV, false>), dim3(rows_grid(rows)), dim3(256), 0, s, op, (const T*)x, ldx,
-                       (T*)y, ldy, rows, cols, crow, vec);
-}
+// Rows that the one-wavefront kernels of this file take: aligned ones whose
+// columns they hold without a remainder (the same speed as rows_reg.hip's,
+// and the packed outputs build on them), and those under 256 columns, where
+// rows_reg.hip's 16-byte vectors leave lanes idle (fp16 8192 x 64: softmax
+// 4.4 us here, 5.3 there).  The others are faster there: softmax 4096 x 777
+// 11.4 -> 8.0 us in fp32 and 12.5 -> 6.4 us in fp16, 2047 x 50257 fp32
+// 340 -> 182 us (4.5 TB/s), layer_norm 512 x 16000 fp32 67 -> 15 us.
+bool wave_row_ok(int64_t cols, bool vec) { return cols < 256 || (vec && cols <= 2048 && cols % 256 == 0); }
 
 template <typename T>
 void sm_launch(int op, const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, int64_t cols, int64_t crow,
                hipStream_t s) {
-  bool vec = vec16_ok(x, ldx, sizeof(T)) && vec16_ok(y, ldy, sizeof(T));
-  switch ((cols + 255) / 256) {
-    case 1: sm_nv<T, 1>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 2: sm_nv<T, 2>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 3: sm_nv<T, 3>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 4: sm_nv<T, 4>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 5: sm_nv<T, 5>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 6: sm_nv<T, 6>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 7: sm_nv<T, 7>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    case 8: sm_nv<T, 8>(op, x, ldx, y, ldy, rows, cols, crow, vec, s); break;
-    default:
-      hipLaunchKernelGGL((softmax_block<T>), dim3((unsigned)rows), dim3(256), 0, s, op, (const T*)x, ldx, (T*)y, ldy,
-                         cols, crow);
+  const bool vec = vec16_ok(x, ldx, sizeof(T)) && vec16_ok(y, ldy, sizeof(T));
+#define AGPU_SM(NV, FULL)                                                                                       \
+  hipLaunchKernelGGL((softmax_wave<T, NV, FULL>), dim3(rows_grid(rows)), dim3(256), 0, s, op, (const T*)x, ldx, \
+                     (T*)y, ldy, rows, cols, crow, vec)
+  if (cols < 256) {
+    AGPU_SM(1, false);
+  } else if (wave_row_ok(cols, vec)) {
+    switch (cols / 256) {
+      case 1: AGPU_SM(1, true); break;
+      case 2: AGPU_SM(2, true); break;
+      case 3: AGPU_SM(3, true); break;
+      case 4: AGPU_SM(4, true); break;
+      case 5: AGPU_SM(5, true); break;
+      case 6: AGPU_SM(6, true); break;
+      case 7: AGPU_SM(7, true); break;
+      default: AGPU_SM(8, true);
+    }
+  } else {
+    hipLaunchKernelGGL((softmax_block<T>), dim3((unsigned)rows), dim3(256), 0, s, op, (const T*)x, ldx, (T*)y, ldy,
+                       cols, crow);
   }
-}
-
-template <typename T, int NV>
-void ln_nv(const void* x, int64_t ldx, const void* g, const void* b, void* y, int64_t rows, int64_t cols, float eps,
-           bool vec, hipStream_t s) {
-  if (vec && cols == NV * 256)
-    hipLaunchKernelGGL((layer_norm_wave<T, NV, true>), dim3(rows_grid(rows)), dim3(256), 0, s, (const T*)x, ldx,
-                       (const T*)g, (const T*)b, (T*)y, rows, cols, eps, vec);
-  else
-    hipLaunchKernelGGL((layer_norm_wave<T, NV, false>), dim3(rows_grid(rows)), dim3(256), 0, s, (const T*)x, ldx,
-                       (const T*)g, (const T*)b, (T*)y, rows, cols, eps, vec);
+#undef AGPU_SM
 }
 
 template <typename T>
 void ln_launch(const void* x, int64_t ldx, const void* g, const void* b, void* y, int64_t rows, int64_t cols,
                float eps, hipStream_t s) {
-  bool vec = vec16_ok(x, ldx, sizeof(T)) && vec16_ok(y, cols, sizeof(T)) && vec16_ok(g, 0, sizeof(T)) &&
-             vec16_ok(b, 0, sizeof(T));
-  switch ((cols + 255) / 256) {
-    case 1: ln_nv<T, 1>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 2: ln_nv<T, 2>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 3: ln_nv<T, 3>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 4: ln_nv<T, 4>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 5: ln_nv<T, 5>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 6: ln_nv<T, 6>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 7: ln_nv<T, 7>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    case 8: ln_nv<T, 8>(x, ldx, g, b, y, rows, cols, eps, vec, s); break;
-    default:
-      hipLaunchKernelGGL((layer_norm_block<T>), dim3((unsigned)rows), dim3(256), 0, s, (const T*)x, ldx, (const T*)g,
-                         (const T*)b, (T*)y, cols, eps);
+  const bool vec = vec16_ok(x, ldx, sizeof(T)) && vec16_ok(y, cols, sizeof(T)) && vec16_ok(g, 0, sizeof(T)) &&
+                   vec16_ok(b, 0, sizeof(T));
+#define AGPU_LN(NV, FULL)                                                                                       \
+  hipLaunchKernelGGL((layer_norm_wave<T, NV, FULL>), dim3(rows_grid(rows)), dim3(256), 0, s, (const T*)x, ldx,  \
+                     (const T*)g, (const T*)b, (T*)y, rows, cols, eps, vec)
+  if (cols < 256) {
+    AGPU_LN(1, false);
+  } else if (wave_row_ok(cols, vec)) {
+    switch (cols / 256) {
+      case 1: AGPU_LN(1, true); break;
+      case 2: AGPU_LN(2, true); break;
+      case 3: AGPU_LN(3, true); break;
+      case 4: AGPU_LN(4, true); break;
+      case 5: AGPU_LN(5, true); break;
+      case 6: AGPU_LN(6, true); break;
+      case 7: AGPU_LN(7, true); break;
+      default: AGPU_LN(8, true);
+    }
+  } else {
+    hipLaunchKernelGGL((layer_norm_block<T>), dim3((unsigned)rows), dim3(256), 0, s, (const T*)x, ldx, (const T*)g,
+                       (const T*)b, (T*)y, cols, eps);
   }
+#undef AGPU_LN
 }
 
 struct LnbArgs {
@@ -1124,14 +1129,24 @@ void softmax_rows(int op, DType dt, const void* x, int64_t ldx, void* y, int64_t
                   int64_t cols, int64_t causal_rows, hipStream_t s) {
   if (rows == 0 || cols == 0) return;
   if (causal_rows <= 0) causal_rows = rows;
-  AGPU_FLOAT_SWITCH(dt, sm_launch<T>(op, x, ldx, y, ldy, rows, cols, causal_rows, s));
+  if (!wave_row_ok(cols, vec16_ok(x, ldx, dtype_size(dt)) && vec16_ok(y, ldy, dtype_size(dt))) &&
+      reg_row_ok(dt, rows, cols))
+    softmax_reg_rows(op, dt, x, ldx, y, ldy, rows, cols, causal_rows, s);
+  else
+    AGPU_FLOAT_SWITCH(dt, sm_launch<T>(op, x, ldx, y, ldy, rows, cols, causal_rows, s));
   check_launch("softmax_rows");
 }
 
 void layer_norm(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y,
                 int64_t rows, int64_t cols, float eps, hipStream_t s) {
   if (rows == 0 || cols == 0) return;
-  AGPU_FLOAT_SWITCH(dt, ln_launch<T>(x, ldx, gamma, beta, y, rows, cols, eps, s));
+  const size_t es = dtype_size(dt);
+  if (!wave_row_ok(cols, vec16_ok(x, ldx, es) && vec16_ok(y, cols, es) && vec16_ok(gamma, 0, es) &&
+                             vec16_ok(beta, 0, es)) &&
+      reg_row_ok(dt, rows, cols))
+    layer_norm_reg_rows(dt, x, ldx, gamma, beta, y, rows, cols, eps, s);
+  else
+    AGPU_FLOAT_SWITCH(dt, ln_launch<T>(x, ldx, gamma, beta, y, rows, cols, eps, s));
   check_launch("layer_norm");
 }
 
