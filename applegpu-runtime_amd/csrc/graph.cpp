@@ -35,7 +35,7 @@ enum Op : int {
   OP_LAYER_NORM_BACKWARD, OP_LAYER_NORM_GRADS, OP_GELU_BACKWARD, OP_GELU_TANH_BACKWARD, OP_GELU_EXACT_BACKWARD,
   OP_EMBEDDING_BACKWARD, OP_PACK_WEIGHT_X3, OP_PACK_ROWS_X3, OP_MATMUL_PP, OP_ROW_STATS_X3, OP_MATMUL_PP_NORM,
   OP_LINEAR_BACKWARD_SGD, OP_LINEAR_MSE_BACKWARD_SGD, OP_MLP2_SGD_STEP, OP_LINEAR_BACKWARD_SGD_PAIR,
-  OP_LINEAR_RELU_MSE_BACKWARD_SGD,
+  OP_LINEAR_RELU_MSE_BACKWARD_SGD, OP_ATTENTION_BACKWARD,
   OP_COUNT
 };
 
@@ -57,7 +57,7 @@ static const char* kNames[OP_COUNT] = {
     "layer_norm_backward", "layer_norm_grads", "gelu_backward", "gelu_tanh_backward", "gelu_exact_backward",
     "embedding_backward", "pack_weight_x3", "pack_rows_x3", "matmul_pp", "row_stats_x3", "matmul_pp_norm",
     "linear_backward_sgd_", "linear_mse_backward_sgd_", "mlp2_sgd_step_", "linear_backward_sgd_pair_",
-    "linear_relu_mse_backward_sgd_",
+    "linear_relu_mse_backward_sgd_", "attention_backward",
 };
 
 int op_code(const char* name) {
@@ -76,7 +76,7 @@ int op_code(const char* name) {
 }
 const char* op_name(int code) { return code >= 0 && code < OP_COUNT ? kNames[code] : "?"; }
 int op_outputs(int code) {
-  if (code == OP_LAYER_NORM_GRADS) return 3;
+  if (code == OP_LAYER_NORM_GRADS || code == OP_ATTENTION_BACKWARD) return 3;
   return code == OP_QUANTIZE_PER_ROW || code == OP_MSE_LOSS_GRAD ? 2 : 1;
 }
 
@@ -206,6 +206,16 @@ std::vector<TensorP> run_op(int code, const std::vector<TensorP>& in, const std:
       // optional f[0]: the softmax scale (default 1/sqrt(D))
       need(in, 3, code);
       return {attention(in[0], in[1], in[2], code == OP_ATTENTION_CAUSAL, false, f.empty() ? 0.f : (float)f[0])};
+    case OP_ATTENTION_BACKWARD: {
+      // (grad, q, k, v), f[0]: scale, iv: causal, then whether dq, dk and dv
+      // are needed; one that is not comes back as [0]
+      need(in, 4, code);
+      auto r = attention_backward(in[0], in[1], in[2], in[3], ip(iv, 0, code) != 0, (float)fp(f, 0, code),
+                                  ip(iv, 1, code) != 0, ip(iv, 2, code) != 0, ip(iv, 3, code) != 0);
+      for (TensorP& t : r)
+        if (!t) t = full(in[0]->dtype, {0}, 0.f);
+      return r;
+    }
     case OP_WHERE: need(in, 3, code); return {where(in[0], in[1], in[2])};
     case OP_MASKED_FILL: need(in, 2, code); return {masked_fill(in[0], in[1], (float)fp(f, 0, code))};
     case OP_TRIU: need(in, 1, code); return {tri(in[0], true, iv.empty() ? 0 : iv[0])};

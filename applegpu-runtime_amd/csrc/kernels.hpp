@@ -413,6 +413,22 @@ struct Attn {
   const void* qb = nullptr; const void* kb = nullptr; const void* vb = nullptr;
 };
 bool attention_supported(const Attn& a);
+// The backward of fp32 attention (attention_bwd.hip): the gradients of q, k
+// and v (contiguous [B, H, T, D]; dq, or dk and dv together, may be null)
+// from the output's gradient.  `stats` is a workspace of 2 * B * H * Tq
+// floats.  Rows need 16-byte alignment (attention_backward_rows_ok) and unit
+// stride along D.
+struct AttnBwd {
+  struct Rows { const void* p = nullptr; int64_t sb = 0, sh = 0, st = 0; };
+  int64_t B = 1, H = 1, Tq = 0, Tk = 0, D = 0;
+  Rows q, k, v, go;
+  void *stats = nullptr, *dq = nullptr, *dk = nullptr, *dv = nullptr;
+  bool causal = false;
+  float scale = 1.f;
+};
+bool attention_backward_ok(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t D);
+bool attention_backward_rows_ok(const void* p, int64_t sb, int64_t sh, int64_t st);
+void attention_backward(const AttnBwd& a, hipStream_t s);
 // Whether attention can read Q/K/V as projection partials (fp32 MFMA kernel:
 // d = 64 or 128, 16-byte aligned rows).
 bool attention_partials_ok(const Attn& a);

@@ -1552,6 +1552,12 @@ TensorP linear_int8(const TensorP& x, const TensorP& q, const TensorP& scale) {
 }
 
 // ── attention ──────────────────────────────────────────────────────────────
+// Leading dims of an attention operand as (batch, head) strides.
+static void lead_strides(const Tensor& t, int64_t* sb, int64_t* sh) {
+  *sb = t.ndim == 4 ? t.strides[0] : 0;
+  *sh = t.ndim == 4 ? t.strides[1] : t.ndim == 3 ? t.strides[0] : 0;
+}
+
 TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool causal, bool out_layout_thd,
                   float scale_arg) {
   const char* name = causal ? "attention_causal" : "attention";
@@ -1588,12 +1594,6 @@ TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool ca
     TensorP p = softmax(s, causal ? k::kSoftmaxCausal : k::kSoftmax);
     return matmul(p, v);
   }
-  // leading dims -> (B, H)
-  auto lead_strides = [](const Tensor& t, int64_t* sb, int64_t* sh) {
-    if (t.ndim == 2) { *sb = 0; *sh = 0; }
-    else if (t.ndim == 3) { *sb = 0; *sh = t.strides[0]; }
-    else { *sb = t.strides[0]; *sh = t.strides[1]; }
-  };
   a.B = q->ndim == 4 ? q->shape[0] : 1;
   a.H = q->ndim == 4 ? q->shape[1] : (q->ndim == 3 ? q->shape[0] : 1);
   a.q = q->data(); lead_strides(*q, &a.q_sb, &a.q_sh); a.q_st = q->strides[q->ndim - 2];
@@ -1623,6 +1623,62 @@ TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool ca
   a.o_st = out->strides[out->ndim - 2];
   LAUNCH k::attention(a, rt().stream());
   return out;
+}
+
+// (dq, dk, dv) of attention(q, k, v) for the output's gradient; one that is
+// not needed comes back null.  fp32 heads that attention_bwd.hip takes run
+// there; others form P = softmax(q k^T s) (top-left causal mask, as torch's
+// is_causal), dV = P^T dO, dS = softmax_backward(dO V^T, P), dQ = s dS K and
+// dK = s dS^T Q on the GEMMs.
+std::vector<TensorP> attention_backward(const TensorP& go, const TensorP& q, const TensorP& kk, const TensorP& v,
+                                        bool causal, float scale, bool need_q, bool need_k, bool need_v) {
+  const int nd = q->ndim;
+  bool fused = q->dtype == DType::F32 && kk->dtype == DType::F32 && v->dtype == DType::F32 &&
+               go->dtype == DType::F32 && nd >= 2 && nd <= 4 && kk->ndim == nd && v->dims() == kk->dims() &&
+               go->dims() == q->dims();
+  for (int i = 0; fused && i < nd; ++i) fused = i == nd - 2 || kk->shape[i] == q->shape[i];
+  k::AttnBwd a;
+  if (fused) {
+    a.B = nd == 4 ? q->shape[0] : 1;
+    a.H = nd == 4 ? q->shape[1] : nd == 3 ? q->shape[0] : 1;
+    a.Tq = q->shape[nd - 2]; a.Tk = kk->shape[nd - 2]; a.D = q->shape[nd - 1];
+    fused = k::attention_backward_ok(a.B, a.H, a.Tq, a.Tk, a.D);
+  }
+  if (!fused) {
+    TensorP p = softmax(unary(k::kScale, matmul(q, kk, false, true), scale), causal ? k::kSoftmaxCausal : k::kSoftmax);
+    TensorP dq, dk, dv;
+    if (need_v) dv = matmul(p, go, true, false);
+    TensorP ds = softmax_backward(matmul(go, v, false, true), p);
+    if (need_q) dq = unary(k::kScale, matmul(ds, kk, false, false), scale);
+    if (need_k) dk = unary(k::kScale, matmul(ds, q, true, false), scale);
+    return {dq, dk, dv};
+  }
+  a.causal = causal;
+  a.scale = scale;
+  TensorP dq, dk, dv;
+  if (need_q) dq = alloc_out(DType::F32, q->dims());
+  if (need_k || need_v) { dk = alloc_out(DType::F32, kk->dims()); dv = alloc_out(DType::F32, v->dims()); }
+  if (meta_mode()) return {dq, need_k ? dk : nullptr, need_v ? dv : nullptr};
+  std::vector<TensorP> keep;  // copies of operands whose rows the kernel cannot read in place
+  auto rows = [&](const TensorP& t) {
+    k::AttnBwd::Rows r;
+    lead_strides(*t, &r.sb, &r.sh);
+    r.st = t->strides[nd - 2];
+    keep.push_back(t->strides[nd - 1] == 1 && k::attention_backward_rows_ok(t->data(), r.sb, r.sh, r.st)
+                       ? t : materialize(t));
+    const Tensor& c = *keep.back();
+    lead_strides(c, &r.sb, &r.sh);
+    r.st = c.strides[nd - 2];
+    r.p = c.data();
+    return r;
+  };
+  a.q = rows(q); a.k = rows(kk); a.v = rows(v); a.go = rows(go);
+  BufferP stats = scratch((size_t)(2 * a.B * a.H * a.Tq) * sizeof(float));
+  a.stats = stats->ptr;
+  if (dq) a.dq = dq->data();
+  if (dk) { a.dk = dk->data(); a.dv = dv->data(); }
+  k::attention_backward(a, rt().stream());
+  return {dq, need_k ? dk : nullptr, need_v ? dv : nullptr};
 }
 
 TensorP attention_rows_x3(const TensorP& q, const TensorP& kk, const TensorP& v, bool causal, float scale_arg) {

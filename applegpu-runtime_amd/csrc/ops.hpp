@@ -240,6 +240,9 @@ TensorP qkv_attention(const TensorP& x, const TensorP& w, const TensorP& b, int6
 // (crates/core/src/ops.rs:1531-1620).
 TensorP attention(const TensorP& q, const TensorP& k, const TensorP& v, bool causal,
                   bool out_layout_thd = false, float scale = 0.f);
+// (dq, dk, dv) of attention(q, k, v) for the output's gradient.
+std::vector<TensorP> attention_backward(const TensorP& go, const TensorP& q, const TensorP& k, const TensorP& v,
+                                        bool causal, float scale, bool need_q, bool need_k, bool need_v);
 // The same attention (fp32, fused kernel) with its output written as packed
 // x3 rows (pack_rows_x3) of the [B*Tq, H*D] matrix of head-merged query rows:
 // the A operand of the following projection (matmul_pp), never stored in

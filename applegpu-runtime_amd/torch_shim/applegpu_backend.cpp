@@ -627,9 +627,8 @@ ag_sdpa_overrideable(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
           at::Tensor(), at::Tensor()};
 }
 
-// P = softmax(q k^T s) recomputed (top-left causal mask, as torch's
-// is_causal), then dV = P^T dO, dS = softmax_backward(dO V^T, P),
-// dQ = s dS K, dK = s dS^T Q; every product on the device GEMM.
+// One op (fp32: the fused backward kernel; else P recomputed and the products
+// on the device GEMM).
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> ag_sdpa_overrideable_backward(
     const at::Tensor& go, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor&,
     std::array<bool, 4> mask, const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
@@ -637,13 +636,16 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> ag_sdpa_overrideable_
     std::optional<double> scale) {
   TORCH_CHECK(dropout == 0.0, "applegpu fused attention backward: no dropout");
   const double s = sdp_scale(q, scale);
-  at::Tensor sc = run_t("scalar_mul", {run_t("matmul_ex", {q, k}, {}, {0, 1})}, {s});
-  at::Tensor p = run_t(is_causal ? "softmax_causal" : "softmax", {sc});
-  at::Tensor dv = mask[2] ? run_t("matmul_ex", {p, go}, {}, {1, 0}) : at::Tensor();
-  at::Tensor ds = run_t("softmax_backward", {run_t("matmul_ex", {go, v}, {}, {0, 1}), p});
-  at::Tensor dq = mask[0] ? run_t("scalar_mul", {run_t("matmul_ex", {ds, k}, {}, {0, 0})}, {s}) : at::Tensor();
-  at::Tensor dk = mask[1] ? run_t("scalar_mul", {run_t("matmul_ex", {ds, q}, {}, {1, 0})}, {s}) : at::Tensor();
-  return {dq, dk, dv, at::Tensor()};
+  Views vw;
+  uint64_t ins[4] = {vw.of(go), vw.of(q), vw.of(k), vw.of(v)}, outs[3] = {0, 0, 0};
+  const int64_t iv[4] = {is_causal, mask[0], mask[1], mask[2]};
+  if (applegpu_eager_op("attention_backward", ins, 4, &s, 1, iv, 4, outs, 3) != 3) fail_last("attention_backward");
+  at::Tensor g[3];
+  for (int i = 0; i < 3; ++i) {
+    at::Tensor t = wrap(outs[i]);
+    if (mask[i]) g[i] = t;
+  }
+  return {g[0], g[1], g[2], at::Tensor()};
 }
 
 at::Tensor ag_softmax(const at::Tensor& self, int64_t dim, bool half_to_float) {
