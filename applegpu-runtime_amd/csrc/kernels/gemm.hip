@@ -901,7 +901,7 @@ const char* gemm_plan_name(const Gemm& g) {
     return buf;
   }
   if (use_h16(g)) {
-    snprintf(buf, sizeof buf, "h16 256x256 w16");
+    snprintf(buf, sizeof buf, "%s", gemm_h16_name(g, cu_count()));
     return buf;
   }
   if (use_f32s(g)) {
