@@ -806,16 +806,39 @@ __global__ void __launch_bounds__(256) gemm_mf(GArgs p) {
             msk[r] = to_f(((const TC*)p.mask)[b * p.k_sb + (row < p.M ? row : p.M - 1) * p.k_sm + cc]);
           }
         }
+        // the activation and the operands' tests once for the block's 16
+        // outputs, not once for each: the branches cost as much as the stores
+        float v[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t row = r0 + 8 * (r >> 2) + (r & 3);
-          float v = p.alpha * acc[i][j][r] + bias;
-          if (p.act == kActRelu) v = fmaxf(v, 0.f);
-          else if (p.act == kActGelu) v = gelu_tanh(v);
-          else if (p.act == kActGeluExact) v = 0.5f * v * (1.f + erff(v * 0.70710678118654752f));
-          if (p.res) v += res[r];
-          if (p.mask) v = msk[r] > 0.f ? v : 0.f;
-          if (row < p.M && col < p.N) ((TC*)p.C)[b * p.c_sb + row * p.c_sm + col] = from_f<TC>(v);
+        for (int r = 0; r < 16; ++r) v[r] = p.alpha * acc[i][j][r] + bias;
+        if (p.act == kActRelu) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] = fmaxf(v[r], 0.f);
+        } else if (p.act == kActGelu) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] = gelu_tanh(v[r]);
+        } else if (p.act == kActGeluExact) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] = 0.5f * v[r] * (1.f + erff(v[r] * 0.70710678118654752f));
+        }
+        if (p.res) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] += res[r];
+        }
+        if (p.mask) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) v[r] = msk[r] > 0.f ? v[r] : 0.f;
+        }
+        TC* out = (TC*)p.C + b * p.c_sb + col;
+        if (r0 + 27 < p.M && col < p.N) {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) out[(r0 + 8 * (r >> 2) + (r & 3)) * p.c_sm] = from_f<TC>(v[r]);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int64_t row = r0 + 8 * (r >> 2) + (r & 3);
+            if (row < p.M && col < p.N) out[row * p.c_sm] = from_f<TC>(v[r]);
+          }
         }
       }
     return;
