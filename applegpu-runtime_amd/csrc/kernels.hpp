@@ -430,7 +430,7 @@ bool attention_backward_ok(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t
 bool attention_backward_rows_ok(const void* p, int64_t sb, int64_t sh, int64_t st);
 void attention_backward(const AttnBwd& a, hipStream_t s);
 // Whether attention can read Q/K/V as projection partials (fp32 MFMA kernel:
-// d = 64 or 128, 16-byte aligned rows).
+// d = 32, 64 or 128, 16-byte aligned rows).
 bool attention_partials_ok(const Attn& a);
 void attention(const Attn& a, hipStream_t s);
 
