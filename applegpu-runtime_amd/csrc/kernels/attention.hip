@@ -961,8 +961,7 @@ template <typename T>
 static void launch_fa_mfma(const AArgs& p, int64_t D, bool wide, unsigned blocks, hipStream_t s) {
   const dim3 grid(blocks), block(64 * kFaWaves);
   if (D == 32) {
-    if (wide) hipLaunchKernelGGL((flash_attn_mfma<T, 32, 2>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((flash_attn_mfma<T, 32, 1>), grid, block, 0, s, p);
+    hipLaunchKernelGGL((flash_attn_mfma<T, 32, 1>), grid, block, 0, s, p);
   } else if (D == 64) {
     if (wide) hipLaunchKernelGGL((flash_attn_mfma<T, 64, 2>), grid, block, 0, s, p);
     else hipLaunchKernelGGL((flash_attn_mfma<T, 64, 1>), grid, block, 0, s, p);
@@ -1049,9 +1048,12 @@ void attention(const Attn& a, hipStream_t s) {
     return;
   }
   if (attention_mfma_ok(a)) {
-    // 128 query rows per block when that still gives every CU a block
+    // 128 query rows per block when that still gives every CU a block; at
+    // head dim 32 always 64: there the softmax, not the products, takes the
+    // time, and more blocks hide it better (42 heads of 1587 tokens, fp16: 45
+    // us with 128 rows, 38 us with 64)
     const int64_t bh = a.B * a.H;
-    const bool wide = bh * ((a.Tq + 127) / 128) >= 256;
+    const bool wide = a.D != 32 && bh * ((a.Tq + 127) / 128) >= 256;
     const int qb = wide ? 128 : 64;
     p.q_tiles = (int)((a.Tq + qb - 1) / qb);
     const int64_t blocks = bh * p.q_tiles;
