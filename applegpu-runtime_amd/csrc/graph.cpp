@@ -35,7 +35,7 @@ enum Op : int {
   OP_LAYER_NORM_BACKWARD, OP_LAYER_NORM_GRADS, OP_GELU_BACKWARD, OP_GELU_TANH_BACKWARD, OP_GELU_EXACT_BACKWARD,
   OP_EMBEDDING_BACKWARD, OP_PACK_WEIGHT_X3, OP_PACK_ROWS_X3, OP_MATMUL_PP, OP_ROW_STATS_X3, OP_MATMUL_PP_NORM,
   OP_LINEAR_BACKWARD_SGD, OP_LINEAR_MSE_BACKWARD_SGD, OP_MLP2_SGD_STEP, OP_LINEAR_BACKWARD_SGD_PAIR,
-  OP_LINEAR_RELU_MSE_BACKWARD_SGD, OP_ATTENTION_BACKWARD,
+  OP_LINEAR_RELU_MSE_BACKWARD_SGD, OP_ATTENTION_BACKWARD, OP_LAYER_NORM_STATS,
   OP_COUNT
 };
 
@@ -57,7 +57,7 @@ static const char* kNames[OP_COUNT] = {
     "layer_norm_backward", "layer_norm_grads", "gelu_backward", "gelu_tanh_backward", "gelu_exact_backward",
     "embedding_backward", "pack_weight_x3", "pack_rows_x3", "matmul_pp", "row_stats_x3", "matmul_pp_norm",
     "linear_backward_sgd_", "linear_mse_backward_sgd_", "mlp2_sgd_step_", "linear_backward_sgd_pair_",
-    "linear_relu_mse_backward_sgd_", "attention_backward",
+    "linear_relu_mse_backward_sgd_", "attention_backward", "layer_norm_stats",
 };
 
 int op_code(const char* name) {
@@ -76,7 +76,7 @@ int op_code(const char* name) {
 }
 const char* op_name(int code) { return code >= 0 && code < OP_COUNT ? kNames[code] : "?"; }
 int op_outputs(int code) {
-  if (code == OP_LAYER_NORM_GRADS || code == OP_ATTENTION_BACKWARD) return 3;
+  if (code == OP_LAYER_NORM_GRADS || code == OP_ATTENTION_BACKWARD || code == OP_LAYER_NORM_STATS) return 3;
   return code == OP_QUANTIZE_PER_ROW || code == OP_MSE_LOSS_GRAD ? 2 : 1;
 }
 
@@ -139,6 +139,9 @@ std::vector<TensorP> run_op(int code, const std::vector<TensorP>& in, const std:
     case OP_LAYER_NORM:
       need(in, 3, code);
       return {layer_norm(in[0], in[1], in[2], f.empty() ? 1e-5f : (float)f[0])};
+    case OP_LAYER_NORM_STATS:
+      need(in, 3, code);
+      return layer_norm_stats(in[0], in[1], in[2], f.empty() ? 1e-5f : (float)f[0]);
     case OP_SUM: need(in, 1, code); return {row_reduce(k::kRSum, in[0])};
     case OP_MEAN: need(in, 1, code); return {row_reduce(k::kRMean, in[0])};
     case OP_AMAX: need(in, 1, code); return {row_reduce(k::kRAmax, in[0])};

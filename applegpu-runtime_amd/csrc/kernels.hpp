@@ -89,15 +89,17 @@ void fused_chain(DType dt, const ChainProgram& prog, ChainLeaves leaves, void* o
 enum RowOp : int { kSoftmax, kLogSoftmax, kSoftmaxCausal };
 void softmax_rows(int op, DType dt, const void* x, int64_t ldx, void* y, int64_t ldy,
                   int64_t rows, int64_t cols, int64_t causal_rows, hipStream_t s);
-void layer_norm(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta,
-                void* y, int64_t rows, int64_t cols, float eps, hipStream_t s);
+// mean and rstd (both or neither; dt, one per row): also the row's mean and
+// 1 / sqrt(var + eps), which the row's wavefront holds anyway.
+void layer_norm(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y, void* mean,
+                void* rstd, int64_t rows, int64_t cols, float eps, hipStream_t s);
 // The same ops on rows held as 16-byte vectors of any alignment
 // (rows_reg.hip), where reg_row_ok says that the row fits the registers.
 bool reg_row_ok(DType dt, int64_t rows, int64_t cols);
 void softmax_reg_rows(int op, DType dt, const void* x, int64_t ldx, void* y, int64_t ldy, int64_t rows, int64_t cols,
                       int64_t causal_rows, hipStream_t s);
 void layer_norm_reg_rows(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y,
-                         int64_t rows, int64_t cols, float eps, hipStream_t s);
+                         void* mean, void* rstd, int64_t rows, int64_t cols, float eps, hipStream_t s);
 enum RedOp : int { kRSum, kRMean, kRAmax, kRArgmax, kRVar };
 void row_reduce(int op, DType in, DType out, const void* x, int64_t ldx, void* y, int64_t rows,
                 int64_t cols, int correction, hipStream_t s);

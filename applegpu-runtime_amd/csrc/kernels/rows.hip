@@ -256,7 +256,8 @@ __global__ void __launch_bounds__(256) softmax_block(int op, const T* __restrict
 template <typename T, int NV, bool FULL>
 __global__ void __launch_bounds__(256) layer_norm_wave(const T* __restrict__ x, int64_t ldx,
                                                        const T* __restrict__ g, const T* __restrict__ b,
-                                                       T* __restrict__ y, int64_t rows, int64_t cols,
+                                                       T* __restrict__ y, T* __restrict__ mean_out,
+                                                       T* __restrict__ rstd_out, int64_t rows, int64_t cols,
                                                        float eps, bool vec) {
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
@@ -283,6 +284,10 @@ __global__ void __launch_bounds__(256) layer_norm_wave(const T* __restrict__ x, 
   }
   const float var = wave_sum(q) / (float)cols;
   const float inv = 1.f / sqrtf(var + eps);
+  if (mean_out && lane == 0) {
+    mean_out[row] = from_f<T>(mean);
+    rstd_out[row] = from_f<T>(inv);
+  }
   float gv[NV][4], bv[NV][4];
   load_groups<T, NV, FULL>(g, lane, cols, vec, 0.f, gv);
   load_groups<T, NV, FULL>(b, lane, cols, vec, 0.f, bv);
@@ -296,7 +301,8 @@ __global__ void __launch_bounds__(256) layer_norm_wave(const T* __restrict__ x, 
 template <typename T>
 __global__ void __launch_bounds__(256) layer_norm_block(const T* __restrict__ x, int64_t ldx,
                                                         const T* __restrict__ g, const T* __restrict__ b,
-                                                        T* __restrict__ y, int64_t cols, float eps) {
+                                                        T* __restrict__ y, T* __restrict__ mean_out,
+                                                        T* __restrict__ rstd_out, int64_t cols, float eps) {
   __shared__ float sh[4];
   const int64_t row = blockIdx.x;
   const T* xr = x + row * ldx;
@@ -311,6 +317,10 @@ __global__ void __launch_bounds__(256) layer_norm_block(const T* __restrict__ x,
   }
   const float var = block_sum(q, sh) / (float)cols;
   const float inv = 1.f / sqrtf(var + eps);
+  if (mean_out && threadIdx.x == 0) {
+    mean_out[row] = from_f<T>(mean);
+    rstd_out[row] = from_f<T>(inv);
+  }
   for (int64_t c = threadIdx.x; c < cols; c += 256)
     yr[c] = from_f<T>(to_f(g[c]) * (to_f(xr[c]) - mean) * inv + to_f(b[c]));
 }
@@ -1011,13 +1021,13 @@ void sm_launch(int op, const void* x, int64_t ldx, void* y, int64_t ldy, int64_t
 }
 
 template <typename T>
-void ln_launch(const void* x, int64_t ldx, const void* g, const void* b, void* y, int64_t rows, int64_t cols,
-               float eps, hipStream_t s) {
+void ln_launch(const void* x, int64_t ldx, const void* g, const void* b, void* y, void* mean, void* rstd,
+               int64_t rows, int64_t cols, float eps, hipStream_t s) {
   const bool vec = vec16_ok(x, ldx, sizeof(T)) && vec16_ok(y, cols, sizeof(T)) && vec16_ok(g, 0, sizeof(T)) &&
                    vec16_ok(b, 0, sizeof(T));
 #define AGPU_LN(NV, FULL)                                                                                       \
   hipLaunchKernelGGL((layer_norm_wave<T, NV, FULL>), dim3(rows_grid(rows)), dim3(256), 0, s, (const T*)x, ldx,  \
-                     (const T*)g, (const T*)b, (T*)y, rows, cols, eps, vec)
+                     (const T*)g, (const T*)b, (T*)y, (T*)mean, (T*)rstd, rows, cols, eps, vec)
   if (cols < 256) {
     AGPU_LN(1, false);
   } else if (wave_row_ok(cols, vec)) {
@@ -1033,7 +1043,7 @@ void ln_launch(const void* x, int64_t ldx, const void* g, const void* b, void* y
     }
   } else {
     hipLaunchKernelGGL((layer_norm_block<T>), dim3((unsigned)rows), dim3(256), 0, s, (const T*)x, ldx, (const T*)g,
-                       (const T*)b, (T*)y, cols, eps);
+                       (const T*)b, (T*)y, (T*)mean, (T*)rstd, cols, eps);
   }
 #undef AGPU_LN
 }
@@ -1137,16 +1147,16 @@ void softmax_rows(int op, DType dt, const void* x, int64_t ldx, void* y, int64_t
   check_launch("softmax_rows");
 }
 
-void layer_norm(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y,
-                int64_t rows, int64_t cols, float eps, hipStream_t s) {
+void layer_norm(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y, void* mean,
+                void* rstd, int64_t rows, int64_t cols, float eps, hipStream_t s) {
   if (rows == 0 || cols == 0) return;
   const size_t es = dtype_size(dt);
   if (!wave_row_ok(cols, vec16_ok(x, ldx, es) && vec16_ok(y, cols, es) && vec16_ok(gamma, 0, es) &&
                              vec16_ok(beta, 0, es)) &&
       reg_row_ok(dt, rows, cols))
-    layer_norm_reg_rows(dt, x, ldx, gamma, beta, y, rows, cols, eps, s);
+    layer_norm_reg_rows(dt, x, ldx, gamma, beta, y, mean, rstd, rows, cols, eps, s);
   else
-    AGPU_FLOAT_SWITCH(dt, ln_launch<T>(x, ldx, gamma, beta, y, rows, cols, eps, s));
+    AGPU_FLOAT_SWITCH(dt, ln_launch<T>(x, ldx, gamma, beta, y, mean, rstd, rows, cols, eps, s));
   check_launch("layer_norm");
 }
 

@@ -184,7 +184,9 @@ template <typename T, int W, int NV>
 __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) layer_norm_reg(const T* __restrict__ x, int64_t ldx,
                                                                         const T* __restrict__ g,
                                                                         const T* __restrict__ b, T* __restrict__ y,
-                                                                        int64_t rows, int cols, float eps) {
+                                                                        T* __restrict__ mean_out,
+                                                                        T* __restrict__ rstd_out, int64_t rows,
+                                                                        int cols, float eps) {
   __shared__ float sh[W];
   typedef RegRow<T, W, NV> R;
   constexpr int V = R::V;
@@ -213,6 +215,10 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) layer_norm_reg(const T*
     }
   }
   const float inv = 1.f / sqrtf(row_sum<W>(q, sh) / (float)cols + eps);
+  if (mean_out && t == 0) {
+    mean_out[row] = from_f<T>(mean);
+    rstd_out[row] = from_f<T>(inv);
+  }
   r.forget(t);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
@@ -277,11 +283,12 @@ void softmax_reg_rows(int op, DType dt, const void* x, int64_t ldx, void* y, int
 }
 
 void layer_norm_reg_rows(DType dt, const void* x, int64_t ldx, const void* gamma, const void* beta, void* y,
-                         int64_t rows, int64_t cols, float eps, hipStream_t s) {
+                         void* mean, void* rstd, int64_t rows, int64_t cols, float eps, hipStream_t s) {
   AGPU_FLOAT_SWITCH(dt, by_row_bytes<T>(cols * (int64_t)sizeof(T), [&](auto w, auto nv) {
                       hipLaunchKernelGGL((layer_norm_reg<T, w.value, nv.value>), row_blocks(w.value, rows),
                                          dim3(w.value == 1 ? 256 : 64 * w.value), 0, s, (const T*)x, ldx,
-                                         (const T*)gamma, (const T*)beta, (T*)y, rows, (int)cols, eps);
+                                         (const T*)gamma, (const T*)beta, (T*)y, (T*)mean, (T*)rstd, rows,
+                                         (int)cols, eps);
                     }));
 }
 

@@ -484,13 +484,15 @@ TensorP softmax(const TensorP& x, int mode) {
   return out;
 }
 
-TensorP layer_norm(const TensorP& x, const TensorP& g, const TensorP& b, float eps) {
+static std::vector<TensorP> layer_norm_run(const TensorP& x, const TensorP& g, const TensorP& b, float eps,
+                                           bool stats) {
   check_dtype("layer_norm", kFloatOnly, x->dtype);
   if (x->ndim < 1) fail("layer_norm requires at least 1D input");
   const int64_t cols = x->shape[x->ndim - 1];
   if (!(g->ndim == 1 && g->shape[0] == cols)) fail("gamma shape %s must be [%lld]", shape_str(g->dims()).c_str(), (long long)cols);
   if (!(b->ndim == 1 && b->shape[0] == cols)) fail("beta shape %s must be [%lld]", shape_str(b->dims()).c_str(), (long long)cols);
   if (g->dtype != x->dtype || b->dtype != x->dtype) fail("layer_norm: gamma/beta dtype must match the input");
+  if (stats && cols == 0) fail("layer_norm_stats: rows of no columns have no statistics");
   TensorP src = x;
   int64_t rows, ld;
   if (!as_rows(*src, &rows, &ld)) {
@@ -498,9 +500,22 @@ TensorP layer_norm(const TensorP& x, const TensorP& g, const TensorP& b, float e
     as_rows(*src, &rows, &ld);
   }
   TensorP gc = contiguous(g), bc = contiguous(b);
-  TensorP out = alloc_out(x->dtype, x->dims());
-  LAUNCH k::layer_norm(x->dtype, src->data(), ld, gc->data(), bc->data(), out->data(), rows, cols, eps, rt().stream());
-  return out;
+  TensorP out = alloc_out(x->dtype, x->dims()), mean, rstd;
+  if (stats) {
+    mean = alloc_out(x->dtype, {rows});
+    rstd = alloc_out(x->dtype, {rows});
+  }
+  LAUNCH k::layer_norm(x->dtype, src->data(), ld, gc->data(), bc->data(), out->data(), stats ? mean->data() : nullptr,
+                       stats ? rstd->data() : nullptr, rows, cols, eps, rt().stream());
+  return {out, mean, rstd};
+}
+
+TensorP layer_norm(const TensorP& x, const TensorP& g, const TensorP& b, float eps) {
+  return layer_norm_run(x, g, b, eps, false)[0];
+}
+
+std::vector<TensorP> layer_norm_stats(const TensorP& x, const TensorP& g, const TensorP& b, float eps) {
+  return layer_norm_run(x, g, b, eps, true);
 }
 
 // Rows at least this long, when there are at most kLongRowsMax of them,

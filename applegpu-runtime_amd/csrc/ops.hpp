@@ -49,6 +49,9 @@ void copy_into(const TensorP& dst, const TensorP& src);                      // 
 // Rows
 TensorP softmax(const TensorP& x, int mode /* k::RowOp */);
 TensorP layer_norm(const TensorP& x, const TensorP& g, const TensorP& b, float eps);
+// {y, mean, rstd}: layer_norm and, from the same launch, each row's mean and
+// 1 / sqrt(var + eps) ([rows], x's dtype), the statistics its backward takes.
+std::vector<TensorP> layer_norm_stats(const TensorP& x, const TensorP& g, const TensorP& b, float eps);
 TensorP row_reduce(int op /* k::RedOp */, const TensorP& x, int correction = 0);
 TensorP softmax_backward(const TensorP& dy, const TensorP& y);
 // layer_norm backward: {dx} or, with params, {dx, dgamma, dbeta}.
