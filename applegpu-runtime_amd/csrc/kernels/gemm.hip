@@ -822,6 +822,13 @@ static bool use_f32s(const Gemm& g) {
   return tu.cfg < 0 && tu.splits == 0 && tu.f32_mode != kF32Native && gemm_f32_stream_ok(g, cu_count());
 }
 
+// The int8 weight-streaming plan (gemm_i8s.hip), unless a tile configuration
+// or a split count is forced.
+static bool use_i8s(const Gemm& g) {
+  const GemmTune& tu = gemm_tune();
+  return tu.cfg < 0 && tu.splits == 0 && gemm_i8_stream_ok(g);
+}
+
 // The 16-bit large-tile plan (gemm_h16.hip), unless a configuration or a
 // split count is forced.
 static bool use_h16(const Gemm& g) {
@@ -834,6 +841,7 @@ int gemm_splits(const Gemm& g) {
   if (use_outer(g) || use_h16(g)) return 1;
   if (skinny_plan(g, cu_count()).use || thin_kind(g)) return 1;
   if (use_f32s(g)) return gemm_f32_stream_splits(g, cu_count());
+  if (use_i8s(g)) return gemm_i8_stream_splits(g, cu_count());
   const Plan pl = make_plan(g, cu_count());
   return pl.kind == kMf ? pl.splits : 1;
 }
@@ -908,6 +916,10 @@ const char* gemm_plan_name(const Gemm& g) {
     snprintf(buf, sizeof buf, "f32 stream 256 cols splits=%d", gemm_f32_stream_splits(g, cu_count()));
     return buf;
   }
+  if (use_i8s(g)) {
+    snprintf(buf, sizeof buf, "i8 stream 256 cols splits=%d", gemm_i8_stream_splits(g, cu_count()));
+    return buf;
+  }
   Plan pl = make_plan(g, cu_count());
   const char* kind = pl.kind == kGeneric ? "generic" : pl.kind == kNative32 ? "f32-native" : "mf";
   snprintf(buf, sizeof buf, "%s cfg%d %dx%dx%d splits=%d", kind, pl.kind == kMf ? pl.cfg : -1, pl.bm, pl.bn, pl.bk,
@@ -925,6 +937,10 @@ size_t gemm_workspace_bytes(const Gemm& g) {
   const SkinnyPlan sp = skinny_plan(g, cu_count());
   if (sp.use || thin_kind(g)) return 0;
   if (use_f32s(g)) return (size_t)gemm_f32_stream_splits(g, cu_count()) * g.M * g.N * sizeof(float);
+  if (use_i8s(g)) {
+    const int ks = gemm_i8_stream_splits(g, cu_count());
+    return ks > 1 ? (size_t)ks * g.M * g.N * sizeof(float) : 0;
+  }
   Plan pl = make_plan(g, cu_count());
   if (pl.splits <= 1) return 0;
   return (size_t)pl.splits * g.batch * g.M * g.N * sizeof(float);
@@ -1009,6 +1025,19 @@ void gemm(const Gemm& g, void* workspace, hipStream_t s) {
     p.ws = (float*)workspace;
     if (!workspace) fail("gemm: split-K workspace missing");
     gemm_f32_stream(g, p, cu_count(), s);
+    reduce_splits(g, p, s);
+    return;
+  }
+  if (use_i8s(g)) {
+    Plan st{};
+    st.bm = 64;
+    st.bn = 256;
+    st.splits = gemm_i8_stream_splits(g, cu_count());
+    const int64_t phases = (g.K + 127) / 128;
+    st.kps = (phases + st.splits - 1) / st.splits * 128;
+    GArgs p = make_args(g, st);
+    p.ws = (float*)workspace;
+    gemm_i8_stream(g, p, s);
     reduce_splits(g, p, s);
     return;
   }

@@ -937,6 +937,13 @@ void gemm_x3_outer(const Gemm& g, const GArgs& p, void* ws, hipStream_t s);
 bool gemm_f32_stream_ok(const Gemm& g, int cus);
 int gemm_f32_stream_splits(const Gemm& g, int cus);
 void gemm_f32_stream(const Gemm& g, const GArgs& p, int cus, hipStream_t s);
+
+// int8 codes streamed past up to 256 rows of fp32 activations
+// (gemm_i8s.hip): the codes become bf16 exactly, two products instead of
+// three, the column's scale once on the sum.
+bool gemm_i8_stream_ok(const Gemm& g);
+int gemm_i8_stream_splits(const Gemm& g, int cus);
+void gemm_i8_stream(const Gemm& g, const GArgs& p, hipStream_t s);
 bool gemm_x3_outer2_ok(const Gemm& g0, const Gemm& g1);
 void gemm_x3_outer2(const Gemm& g0, const GArgs& p0, void* ws0, const Gemm& g1, const GArgs& p1, void* ws1,
                     hipStream_t s);
