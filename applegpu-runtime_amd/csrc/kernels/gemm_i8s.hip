@@ -2,18 +2,18 @@
 // scale per output column (C[m][n] = scale[n] sum_k A[m][k] q[n][k]): each
 // code is read once, straight into registers, and becomes a bf16 there.
 //
-// Bound by the codes' bytes at few rows, by the matrix cores and LDS beyond
-// 64.  A code (-128 .. 127) is exact in bf16, so the fp32 sum needs two
-// products, A's hi and lo halves times the code, and the scale once at the
-// end; dequantizing first takes three products of split operands, a rounding
-// more, and an LDS round trip of the weights.  Figures at the dispatch rule
-// below.
+// Bound by the requests that a CU has in flight (8192 x 8192 codes: 19 us at
+// one row, 3.5 TB/s; 30 at 64 rows, beside A's loads and splits).  A code
+// (-128 .. 127) is exact in bf16, so the fp32 sum needs two products, A's hi
+// and lo halves times the code, and the scale once at the end; dequantizing
+// first takes three products of split operands, a rounding more, and an LDS
+// round trip of the weights.  (Sums of values past 2^121 can overflow before
+// the scale is applied.)  Figures at the dispatch rule below.
 //
 // A block of 8 wavefronts owns 256 columns and 32 RS rows over one of KS
 // ranges of K.  Wavefront w takes 64 columns (strip w % 4) of one half (w / 4)
-// of the k: two column strips for each fragment of A that it reads, since at
-// one strip the fragments take LDS as long as the products take the matrix
-// cores.  A phase is 128 k: of its half, lane l holds 32 codes from 32 (l / 32)
+// of the k: two column strips for each fragment of A that it reads, half the
+// LDS reads of one strip (64 rows took the same time with one).  A phase is 128 k: of its half, lane l holds 32 codes from 32 (l / 32)
 // of the columns l % 32 and 32 + l % 32, four 16-byte loads, requested two
 // phases ahead (64 KB in flight a block).  Step t of a half multiplies codes
 // 8 t .. + 7, so A's fragment of lane l at step t is row l % 32, k 32 (l / 32)
@@ -288,9 +288,9 @@ int gemm_i8_stream_splits(const Gemm& g, int cus) {
 // their larger grids (128 x 768 x 3072 14.6, here 16.5).
 bool gemm_i8_stream_ok(const Gemm& g) {
   return g.dt == DType::F32 && g.b_dt == DType::I8 && g.b_scale && g.batch == 1 && g.a_sk == 1 && g.b_sk == 1 &&
-         g.M >= 1 && g.M <= 256 && g.N >= 1 &&
-         (g.M <= 64 || g.K % 16 != 0 || g.N * g.K >= (4LL << 20)) && g.K >= 16 && g.K < (1LL << 30) && g.alpha == 1.f && !g.bias && !g.residual && !g.mask &&
-         g.act == 0 && !g.b_x3 && !g.a_x3 && !g.b_packed && !g.ln_gamma && !g.c_pk && !g.pln_y && !g.pln_ypk &&
+         g.M >= 1 && g.M <= 256 && g.N >= 1 && g.K >= 16 && g.K < (1LL << 30) &&
+         (g.M <= 64 || g.K % 16 != 0 || g.N * g.K >= (4LL << 20)) && g.alpha == 1.f && !g.bias && !g.residual &&
+         !g.mask && g.act == 0 && !g.b_x3 && !g.a_x3 && !g.b_packed && !g.ln_gamma && !g.c_pk && !g.pln_y && !g.pln_ypk &&
          !g.no_reduce && !g.a_rowsum_acc && !g.rs_out && !g.rs_in && (g.N + kI8Cols - 1) / kI8Cols <= 0x1000000;
 }
 
