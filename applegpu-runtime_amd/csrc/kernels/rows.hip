@@ -166,18 +166,20 @@ __global__ void __launch_bounds__(256) softmax_wave(int op, const T* __restrict_
 #pragma unroll
     for (int j = 0; j < 4; ++j) mx = fmaxf(mx, v[i][j]);
   mx = wave_max(mx);
-  // 16-bit outputs round to 2^-11 or coarser: exp(v - mx) as 2^(v log2 e -
-  // mx log2 e) on the hardware exp2 (about 1 ulp of fp32) is well inside
-  // that; fp32 rows keep the correctly range-reduced expf.
+  // 16-bit outputs round to 2^-11 or coarser: exp(v - mx) on the hardware
+  // exp2 (about 1 ulp of fp32) is well inside that; fp32 rows keep the
+  // correctly range-reduced expf.  The difference is taken first: it is exact
+  // near the maximum whatever the row's magnitude, where v log2 e - mx log2 e
+  // carries the rounding of mx log2 e into every exponent and overflows for a
+  // row of bf16's lowest value.
   constexpr float kLog2e = 1.4426950408889634f;
-  const float mxl = mx * kLog2e;
   float sum = 0.f;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       float e;
-      if constexpr (sizeof(T) == 2) e = __builtin_amdgcn_exp2f(fmaf(v[i][j], kLog2e, -mxl));
+      if constexpr (sizeof(T) == 2) e = __builtin_amdgcn_exp2f((v[i][j] - mx) * kLog2e);
       else e = expf(v[i][j] - mx);
       sum += e;
       if (op != kLogSoftmax) v[i][j] = e;

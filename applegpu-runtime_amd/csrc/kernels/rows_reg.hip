@@ -131,11 +131,13 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) softmax_reg(const T* __
 #pragma unroll
     for (int j = 0; j < V; ++j) mx = fmaxf(mx, to_f(r.v[i].e[j]));
   mx = row_max<W>(mx, sh);
-  // as in softmax_wave: the hardware exp2 for 16-bit rows, expf for fp32
+  // as in softmax_wave: the hardware exp2 of the difference for 16-bit rows,
+  // expf for fp32
   constexpr float kLog2e = 1.4426950408889634f;
-  const float mxl = mx * kLog2e;
+  float one = 1.f;
+  asm("" : "+s"(one));  // v - mx as an fma, which takes an fp16 v as it is (v_fma_mix)
   auto ex = [&](float v) {
-    if constexpr (sizeof(T) == 2) return __builtin_amdgcn_exp2f(fmaf(v, kLog2e, -mxl));
+    if constexpr (sizeof(T) == 2) return __builtin_amdgcn_exp2f(fmaf(v, one, -mx) * kLog2e);
     else return expf(v - mx);
   };
   r.forget(t);
@@ -162,7 +164,9 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) softmax_reg(const T* __
       for (int j = 0; j < V; ++j) r.v[i].e[j] = from_f<T>(to_f(r.v[i].e[j]) - mx - ls);
     }
   } else {
-    const float inv = 1.f / sum;  // one division per row; the fp32 quotient is corrected by its remainder
+    // one division per row; the fp32 quotient is corrected by its remainder,
+    // 16-bit rows take the division into the exponent
+    const float inv = 1.f / sum, ls2 = -__log2f(sum);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       __builtin_amdgcn_sched_barrier(0);
@@ -172,7 +176,7 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) softmax_reg(const T* __
           const float e = r.v[i].e[j], q = e * inv;
           r.v[i].e[j] = fmaf(fmaf(-q, sum, e), inv, q);
         } else {
-          r.v[i].e[j] = from_f<T>(ex(to_f(r.v[i].e[j])) * inv);
+          r.v[i].e[j] = from_f<T>(__builtin_amdgcn_exp2f(fmaf(fmaf(to_f(r.v[i].e[j]), one, -mx), kLog2e, ls2)));
         }
       }
     }

@@ -77,3 +77,37 @@ def test_rows_of_a_wider_tensor(gpu):
     for lo, hi in ((1, 1000), (3, 1203)):
         got = gpu.softmax(gpu.slice(t, 1, lo, hi)).to_numpy().astype(np.float64)
         np.testing.assert_allclose(got, _softmax64(x[:, lo:hi]), rtol=4e-6, atol=0)
+
+
+@pytest.mark.parametrize("dt", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("cols", [64, 300, 512, 2048, 2500, 4099, 16385, 53249, 65537])
+def test_rows_of_large_magnitude(gpu, cols, dt):
+    """Rows of one value (every column masked with the type's lowest value, or
+    with -1e9 or -1e10, and large positive ones), rows half masked, and rows
+    far from zero whose columns differ: the exponents come from differences
+    with the maximum, which are as exact there as around zero."""
+    t, x = _rows(gpu, 10, cols, dt, 7)
+    x = x.astype(np.float32)
+    lowest = {"float32": -3.4028234e38, "float16": -65504.0, "bfloat16": -3.3895314e38}[dt]
+    for r, v in enumerate((lowest, -1e9, -1e10, -1e12, 1e6, -lowest)):
+        x[r] = np.clip(v, lowest, -lowest)
+    x[6, ::2] = lowest
+    x[7, :-1] = lowest
+    x[8] = np.round(x[8]) * 256 + 32768.0        # steps of 256: 16-bit values too
+    x[9] = np.round(x[9]) * 256 - 32768.0
+    t = gpu.cast(gpu.from_numpy(x), dt) if dt != "float32" else gpu.from_numpy(x)
+    x = t.to_numpy().astype(np.float64)
+    p = _softmax64(x)
+    e = x - x.max(-1, keepdims=True)
+    log_p = e - np.log(np.exp(e).sum(-1, keepdims=True))
+    tiny = 2.0 ** -24 if dt == "float16" else 2.0 ** -126   # below the smallest normal value
+    np.testing.assert_allclose(gpu.softmax(t).to_numpy().astype(np.float64), p, rtol=BAR[dt], atol=tiny)
+    got = gpu.log_softmax(t).to_numpy().astype(np.float64)
+    # a log-probability near the type's lowest value may be its infinity
+    far = log_p < lowest * (1 - 2.0 ** -9)
+    assert (got[far] <= lowest * (1 - 2.0 ** -9)).all()
+    np.testing.assert_allclose(got[~far], log_p[~far], rtol=BAR[dt], atol=4e-6)
+    causal = gpu.softmax_causal(t).to_numpy().astype(np.float64)     # row r: its first r + 1 columns
+    for r in range(10):
+        want = np.r_[_softmax64(x[r:r + 1, :r + 1])[0], np.zeros(cols - r - 1)]
+        np.testing.assert_allclose(causal[r], want, rtol=BAR[dt], atol=tiny)
