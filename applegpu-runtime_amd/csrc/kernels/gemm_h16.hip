@@ -42,9 +42,13 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 __device__ __forceinline__ void lds_copy16(__amdgpu_buffer_rsrc_t src, void* l, int voff, int soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (lds_ptr)l, 16, voff, soff, 0, 0);
 }
+// An offset that is past the end of every resource: what is copied from there
+// is zeros.  A resource spans no more than this, however far its tensor
+// reaches (a tile's own rows end before half of it, see gemm_h16_ok).
+constexpr int kPastEnd = 0x7ffffff0;
 // The rows of an operand from `p` on, `bytes` of them.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_resource(const void* p, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(bytes < 0x7fffffffLL ? bytes : 0x7fffffffLL),
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)(bytes < kPastEnd ? bytes : kPastEnd),
                                            0x00020000);
 }
 
@@ -113,7 +117,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
 #pragma unroll
       for (int q = 0; q < LPW; ++q) {
         const int r = (q < LA ? w * LA + q : w * LB + q - LA) * WR + lr;
-        const int v = ((lane % CH) ^ swz(r)) < left ? off[q] + k : 0x7ffffff0;
+        const int v = ((lane % CH) ^ swz(r)) < left ? off[q] + k : kPastEnd;
         lds_copy16(q < LA ? sa : sb, q < LA ? da + q * 512 : db + (q - LA) * 512, v, 0);
       }
       return;

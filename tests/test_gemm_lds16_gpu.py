@@ -74,6 +74,27 @@ def test_row_ranges_of_wider_tensors(gpu):
         _close(got, xs[:, lo:lo + K] @ ws[:, lo:lo + K].T, "float16")
 
 
+@pytest.mark.parametrize("both", [False, True])
+def test_columns_of_a_tensor_past_2_gib(gpu, both):
+    """A last stage of 8 k of rows 2 MiB apart: what lies 2 GiB behind a
+    tile's first row, outside the columns multiplied, is not read as the
+    stage's padding (an infinity there, or finite values on both sides)."""
+    M, ld, K = 1100, 1 << 20, 72
+    big = np.zeros((M, ld), np.float16)
+    big[:, :2 * K] = RNG.standard_normal((M, 2 * K)) * 0.5
+    big[1023, -8:] = 9.0 if both else np.inf     # byte 0x7ffffff0 from the tensor's first row
+    x = gpu.from_numpy(big)
+    xs = big[:, :2 * K].astype(np.float64)
+    del big
+    xv = gpu.slice(x, 1, 0, K)
+    if both:
+        wv, ws = gpu.slice(x, 1, K, 2 * K), xs[:, K:]
+    else:
+        wv, ws = _dev(gpu, RNG.standard_normal((M, K)) * 0.5, "float16")
+    assert _plan(M, M, K).startswith("lds16")
+    _close((xv @ gpu.transpose(wv)).to_numpy(), xs[:, :K] @ ws.T, "float16")
+
+
 def test_declines():
     assert not _plan(1024, 1280, 100).startswith("lds16")    # rows of partial vectors
     assert not _plan(100, 1280, 1280).startswith("lds16")    # too few tiles
