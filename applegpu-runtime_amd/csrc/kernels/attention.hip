@@ -303,11 +303,23 @@ struct FaTile {
     put_v<VP>(Vt, tid, va0, vb0);
     if constexpr (VU > 1) put_v<VP>(Vt, tid + NT, va1, vb1);
   }
+  // Whether this thread's values of V (VU = 1) hold an infinity or a NaN: two
+  // at a time, an exponent of all ones carries into the sign's place.
+  __device__ __forceinline__ bool v_not_finite(int tid) const {
+    static_assert(VU == 1, "one pair of chunks");
+    constexpr uint32_t one = std::is_same<T, half_t>::value ? 0x04000400u : 0x00800080u;
+    uint32_t c = 0;
+    for (const uint32_t w : {va0.x, va0.y, va0.z, va0.w, vb0.x, vb0.y, vb0.z, vb0.w}) c |= (w & 0x7fff7fffu) + one;
+    return (c & 0x80008000u) != 0 && tid < VT;
+  }
 };
 
-//
-// D = 32 keeps its probabilities to fp32's precision, as the scalar kernel did
-// that took it before: hi + lo in the input type, two products with V.
+// D = 32 keeps its probabilities to fp32's precision, as the scalar kernel
+// does: hi + lo in the input type, two products with V.  And as there, an
+// infinite or NaN value of V reaches the queries that see its key, as itself,
+// and no others: a tile that holds one (its stager says so) is summed key by
+// key, since the products would make NaN of it with a lo or a masked
+// probability of zero.
 template <typename T, int D, int QG>
 __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_mfma(AArgs p) {
   constexpr bool PS = D == 32;
@@ -320,6 +332,7 @@ __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_mfma(AArgs p) {
   constexpr int DT = D / 16;              // 16-dim tiles of O^T
   __shared__ __attribute__((aligned(16))) T Ks[2][kFaKeys * KP];
   __shared__ __attribute__((aligned(16))) T Vt[2][D * VP];
+  __shared__ int v_special[2];  // PS: the last tile in this buffer whose V is not all finite
 
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
@@ -369,6 +382,11 @@ __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_mfma(AArgs p) {
   if (ntiles > 0) {
     FaTile<T, D> t0;
     t0.load(K, V, p, 0, tid);
+    if constexpr (PS) {
+      if (tid < 2) v_special[tid] = -1;
+      __syncthreads();
+      if (t0.v_not_finite(tid)) v_special[0] = 0;
+    }
     t0.template store<KP, VP>(Ks[0], Vt[0], tid);
   }
   __syncthreads();
@@ -388,6 +406,7 @@ __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_mfma(AArgs p) {
 
     const T* Kb = Ks[buf];
     const T* Vb = Vt[buf];
+    const bool special = PS && __builtin_amdgcn_readfirstlane(v_special[buf]) == it;
     f32x4 st[QG][4];
 #pragma unroll
     for (int gi = 0; gi < QG; ++gi)
@@ -429,25 +448,49 @@ __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_mfma(AArgs p) {
           ps += pv;
           const T ph = (T)pv;
           pf[gi][t >> 1][4 * (t & 1) + r] = ph;
-          if constexpr (PS) pl[gi][t >> 1][4 * (t & 1) + r] = (T)(pv - (float)ph);
+          if constexpr (PS) {
+            pl[gi][t >> 1][4 * (t & 1) + r] = (T)(pv - (float)ph);
+            st[gi][t][r] = pv;
+          }
         }
       ls[gi] = ls[gi] * alpha + ps;
 #pragma unroll
       for (int u = 0; u < DT; ++u) acc[gi][u] *= alpha;
     }
+    if (special) {
 #pragma unroll
-    for (int u = 0; u < DT; ++u)
+      for (int gi = 0; gi < QG; ++gi)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const V8 a = *(const V8*)&Vb[(16 * u + l16) * VP + 32 * s + 8 * g];
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int gi = 0; gi < QG; ++gi) {
-          if constexpr (PS) acc[gi][u] = FaMfma<T>::run(a, pl[gi][s], acc[gi][u]);
-          acc[gi][u] = FaMfma<T>::run(a, pf[gi][s], acc[gi][u]);
+          for (int r = 0; r < 4; ++r)
+#pragma unroll 1
+            for (int x = 0; x < 4; ++x) {  // the query's lanes in turn: key 16 t + 4 x + r
+              const int c = 16 * t + 4 * x + r;
+              const float pv = __shfl(st[gi][t][r], 16 * x + l16, 64);
+              if (j0 + c >= lim[gi]) continue;
+#pragma unroll
+              for (int u = 0; u < DT; ++u)
+#pragma unroll
+                for (int y = 0; y < 4; ++y) acc[gi][u][y] += pv * to_f(Vb[(16 * u + 4 * g + y) * VP + fa_vpos(c)]);
+            }
+    } else {
+#pragma unroll
+      for (int u = 0; u < DT; ++u)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const V8 a = *(const V8*)&Vb[(16 * u + l16) * VP + 32 * s + 8 * g];
+#pragma unroll
+          for (int gi = 0; gi < QG; ++gi) {
+            if constexpr (PS) acc[gi][u] = FaMfma<T>::run(a, pl[gi][s], acc[gi][u]);
+            acc[gi][u] = FaMfma<T>::run(a, pf[gi][s], acc[gi][u]);
+          }
         }
-      }
+    }
     // the LDS stores into the other buffer stay after this tile's LDS reads
     asm volatile("" ::: "memory");
+    if constexpr (PS)
+      if (nx.v_not_finite(tid)) v_special[buf ^ 1] = it + 1;
     nx.template store<KP, VP>(Ks[buf ^ 1], Vt[buf ^ 1], tid);
     __syncthreads();
   };
@@ -626,6 +669,10 @@ __device__ __forceinline__ void fa32_store(const AArgs& p, int64_t b, int64_t h,
 // each wavefront then does a quarter of the serial work.  At D = 64 that
 // case runs flash_attn_f32_kr below instead, with its operands in registers.
 // NSP > 0: Q, K and V are read as split-K partials plus bias (ld_part4).
+// D = 32 keeps the scalar kernel's meaning of an infinite or NaN value of V,
+// as in flash_attn_mfma: here only masked probabilities, of zero, could make
+// another NaN of it, so only masked tiles look at their values (each wavefront
+// at its own keys') and are summed key by key.
 template <int D, bool KSPLIT, int NSP>
 __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_f32(AArgs p) {
   static_assert(D % 32 == 0, "d must be a multiple of 32");
@@ -756,25 +803,54 @@ __global__ void __launch_bounds__(64 * kFaWaves) flash_attn_f32(AArgs p) {
     ls = ls * alpha + ps;
 #pragma unroll
     for (int u = 0; u < DT; ++u) acc[u] *= alpha;
+    bool special = false;
+    if constexpr (D == 32 && MASK) {
+      uint32_t top = 0;  // of the lane's V operands, without their signs
 #pragma unroll
-    for (int ti = 0; ti < NT; ++ti)
+      for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float* vr = Vb + (16 * (tw + ti) + 4 * g + r) * KP + DT * l16;
-        float a[DT];
-        if constexpr (DT == 2) {
-          const float2 x = *(const float2*)vr;
-          a[0] = x.x; a[1] = x.y;
-        } else {
-#pragma unroll
-          for (int u = 0; u < DT; u += 4) {
-            const float4 x = *(const float4*)(vr + u);
-            a[u] = x.x; a[u + 1] = x.y; a[u + 2] = x.z; a[u + 3] = x.w;
-          }
+        for (int r = 0; r < 4; ++r) {
+          const uint2 x = *(const uint2*)(Vb + (16 * (tw + ti) + 4 * g + r) * KP + DT * l16);
+          top = max(top, max(x.x & 0x7fffffffu, x.y & 0x7fffffffu));
         }
+      special = __any(top >= 0x7f800000u);
+    }
+    if (special) {
 #pragma unroll
-        for (int u = 0; u < DT; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], st[ti][r], acc[u], 0, 0, 0);
-      }
+      for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll 1
+          for (int x = 0; x < 4; ++x) {  // the query's lanes in turn
+            const int c = 16 * (tw + ti) + 4 * x + r;
+            const float pv = __shfl(st[ti][r], 16 * x + l16, 64);
+            if (j0 + c >= lim) continue;
+#pragma unroll
+            for (int u = 0; u < DT; ++u)
+#pragma unroll
+              for (int y = 0; y < 4; ++y) acc[u][y] += pv * Vb[c * KP + DT * (4 * g + y) + u];
+          }
+    } else {
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float* vr = Vb + (16 * (tw + ti) + 4 * g + r) * KP + DT * l16;
+          float a[DT];
+          if constexpr (DT == 2) {
+            const float2 x = *(const float2*)vr;
+            a[0] = x.x; a[1] = x.y;
+          } else {
+#pragma unroll
+            for (int u = 0; u < DT; u += 4) {
+              const float4 x = *(const float4*)(vr + u);
+              a[u] = x.x; a[u + 1] = x.y; a[u + 2] = x.z; a[u + 3] = x.w;
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < DT; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], st[ti][r], acc[u], 0, 0, 0);
+        }
+    }
 #define AGPU_FA32_ST(I)                                                                    \
     if constexpr (I < NU) {                                                                \
       const int e = tid + 64 * kFaWaves * I;                                               \

@@ -56,3 +56,35 @@ def test_heads_of_a_projection(gpu, dt):
         y = gpu.matmul_pp(gpu.pack_rows_x3(merged), T, gpu.pack_weight_x3(w), 96).to_numpy().astype(np.float64)
         ref = want @ ws
         assert np.linalg.norm(y - ref) <= 1e-5 * np.linalg.norm(ref)   # the split products' 2^-17
+
+
+@pytest.mark.parametrize("dt", list(BAR))
+@pytest.mark.parametrize("B,H,Tq,Tk,causal", [(1, 1, 1, 1, True), (1, 2, 70, 70, True), (1, 2, 70, 130, False),
+                                              (1, 2, 200, 200, True), (2, 70, 130, 130, True), (2, 70, 130, 90, False)])
+def test_infinite_and_nan_values(gpu, dt, B, H, Tq, Tk, causal):
+    """A key's infinite or NaN value reaches the queries that see the key, as
+    itself, and no others: at the first and the last key, inside a tile and on
+    the causal diagonal, beside finite ones in the same row."""
+    a = RNG.standard_normal((B, H, Tk, 32))
+    a[0, 0, 0, 3] = np.inf
+    a[0, 0, Tk // 2, 5] = -np.inf
+    a[0, 0, Tk // 3, 17] = np.nan
+    a[0, 0, Tk - 1, 8:16] = np.inf
+    a[-1, -1, Tk // 2, 30] = np.inf
+    a[-1, -1, Tk - 1, 30] = -np.inf               # both signs: NaN where both are seen
+    (q, qs), (k, ks) = (_dev(gpu, RNG.standard_normal((B, H, t, 32)), dt) for t in (Tq, Tk))
+    v, vs = _dev(gpu, a, dt)
+    got = (gpu.attention_causal if causal else gpu.attention)(q, k, v).to_numpy().astype(np.float64)
+    want = np.empty((B, H, Tq, 32))
+    see = np.tril(np.ones((Tq, Tk), bool)) if causal else np.ones((Tq, Tk), bool)
+    s = np.where(see, qs @ np.swapaxes(ks, -1, -2) / np.sqrt(32.0), -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    with np.errstate(invalid="ignore"):
+        for i in range(Tq):
+            want[:, :, i] = (p[:, :, i, see[i], None] * vs[:, :, see[i]]).sum(2)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isposinf(got), np.isposinf(want))
+    np.testing.assert_array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want)
+    assert np.linalg.norm(got[ok] - want[ok]) <= BAR[dt] * np.linalg.norm(want[ok])
