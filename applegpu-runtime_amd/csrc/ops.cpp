@@ -1642,14 +1642,15 @@ TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool ca
 
 // (dq, dk, dv) of attention(q, k, v) for the output's gradient; one that is
 // not needed comes back null.  fp32 heads that attention_bwd.hip takes run
-// there; others form P = softmax(q k^T s) (top-left causal mask, as torch's
+// there, unless the native fp32 products are chosen (it multiplies split
+// operands, as the default GEMMs do); others form P = softmax(q k^T s) (top-left causal mask, as torch's
 // is_causal), dV = P^T dO, dS = softmax_backward(dO V^T, P), dQ = s dS K and
 // dK = s dS^T Q on the GEMMs.
 std::vector<TensorP> attention_backward(const TensorP& go, const TensorP& q, const TensorP& kk, const TensorP& v,
                                         bool causal, float scale, bool need_q, bool need_k, bool need_v) {
   const int nd = q->ndim;
   bool fused = q->dtype == DType::F32 && kk->dtype == DType::F32 && v->dtype == DType::F32 &&
-               go->dtype == DType::F32 && nd >= 2 && nd <= 4 && kk->ndim == nd && v->dims() == kk->dims() &&
+               go->dtype == DType::F32 && k::gemm_tune().f32_mode != k::kF32Native && nd >= 2 && nd <= 4 && kk->ndim == nd && v->dims() == kk->dims() &&
                go->dims() == q->dims();
   for (int i = 0; fused && i < nd; ++i) fused = i == nd - 2 || kk->shape[i] == q->shape[i];
   k::AttnBwd a;

@@ -110,3 +110,20 @@ def test_same_bits_twice_and_rows_that_never_end(torch_dev):
     c = grads(q)
     assert torch.isnan(c[0][0, 1, 7]).all() and torch.equal(c[0][0, 0], a[0][0, 0])
     assert torch.isnan(c[1][0, 1, 0]).all() and torch.equal(c[1][0, 2], a[1][0, 2])
+
+
+def test_native_fp32_products(torch_dev):
+    """With the native fp32 products chosen, the gradients keep their
+    precision too (split products are 8e-6 off, fp32 sums of 300 terms 1e-6)."""
+    torch = torch_dev
+    from applegpu_runtime._native import lib
+    torch.manual_seed(11)
+    q, k, v, go = (torch.randn(2, 3, 300, 64) for _ in range(4))
+    assert lib.applegpu_ffi_gemm_tune(1, -1, 0) == 0
+    try:
+        dev = [t.to("applegpu").requires_grad_(True) for t in (q, k, v)]
+        out = torch.nn.functional.scaled_dot_product_attention(*dev, is_causal=True)
+        got = (out,) + torch.autograd.grad(out, dev, go.to("applegpu"))
+        _check(torch, got, _reference(torch, q, k, v, go, True), bar=1e-6)
+    finally:
+        lib.applegpu_ffi_gemm_tune(0, -1, 0)
