@@ -7,8 +7,9 @@
 // (-128 .. 127) is exact in bf16, so the fp32 sum needs two products, A's hi
 // and lo halves times the code, and the scale once at the end; dequantizing
 // first takes three products of split operands, a rounding more, and an LDS
-// round trip of the weights.  (Sums of values past 2^121 can overflow before
-// the scale is applied.)  Figures at the dispatch rule below.
+// round trip of the weights.  Where the sum passes fp32's range before the
+// scale is applied (values past 2^121), that output is summed again in 64
+// bits.  Figures at the dispatch rule below.
 //
 // A block of 8 wavefronts owns 256 columns and 32 RS rows over one of KS
 // ranges of K.  Wavefront w takes 64 columns (strip w % 4) of one half (w / 4)
@@ -236,17 +237,32 @@ __global__ void __launch_bounds__(512, 1) gemm_i8_stream_kernel(GArgs p, int KS)
   float sc = p.b_scale[nc];
   if (!(fabsf(sc) < INFINITY)) sc = NAN;
   float* ws = p.ws + ks * (p.M * p.N);
+  auto put = [&](int64_t row, float v) __attribute__((always_inline)) {
+    if (KS > 1) ws[row * p.N + nc] = v;
+    else ((float*)p.C)[row * p.c_sm + nc] = v;
+  };
+  uint32_t over = 0;  // bit 16 i + r: an output whose sum is not finite
 #pragma unroll
   for (int i = 0; i < RS; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int64_t row = m0 + 32 * i + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
       if (row < p.M) {
-        const float v = ((half ? acc[i][1][r] : acc[i][0][r]) + red[(w ^ 4) * RED + (i * 16 + r) * 64 + lane]) * sc;
-        if (KS > 1) ws[row * p.N + nc] = v;
-        else ((float*)p.C)[row * p.c_sm + nc] = v;
+        const float v = (half ? acc[i][1][r] : acc[i][0][r]) + red[(w ^ 4) * RED + (i * 16 + r) * 64 + lane];
+        put(row, v * sc);
+        if (!(fabsf(v) < INFINITY)) over |= 1u << (16 * i + r);
       }
     }
+  const int kend = min(K, kbeg + (int)p.k_per_split);
+  const int8_t* q = half ? Bn[1] : Bn[0];
+  for (; over; over &= over - 1) {
+    const int e = __builtin_ctz(over);
+    const int64_t row = m0 + 32 * (e >> 4) + 8 * ((e >> 2) & 3) + 4 * (lane >> 5) + (e & 3);
+    const float* a1 = (const float*)p.A + row * p.a_sm;
+    double v = 0;
+    for (int k = kbeg; k < kend; ++k) v += (double)a1[k] * q[k];
+    put(row, (float)(v * sc));
+  }
 }
 
 int i8s_strips(const Gemm& g) { return g.M <= 32 ? 1 : 2; }

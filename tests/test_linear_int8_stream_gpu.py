@@ -60,3 +60,25 @@ def test_special_scales_and_rows(gpu):
     np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
     ok = ~np.isnan(want)
     assert np.linalg.norm(got[ok] - want[ok]) <= 1e-5 * np.linalg.norm(want[ok])
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 40, 128), (20, 64, 300), (64, 512, 2048), (130, 256, 100)])
+def test_sums_past_fp32_before_the_scale(gpu, M, N, K):
+    """Results that fp32 holds come out although the sum of values times codes
+    passes its range on the way, in one range of K, in one of its halves or in
+    the sum of both; a scale of zero gives zero."""
+    x, q, s = _data(M, N, K)
+    s[:] = (RNG.random(N) + 0.5) * 2.0 ** -20
+    s[1 % N] = 0.0
+    x *= 2.0 ** 118                                # 2^118 * 2^7 * sqrt(K) and more
+    x[0, :16] = 2.0 ** 126
+    q[:, :16] = 127
+    got = _run(gpu, x, q, s)
+    want = (x.astype(np.float64) @ q.astype(np.float64).T) * s.astype(np.float64)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got / 2.0 ** 110 - want / 2.0 ** 110) <= 1e-5 * np.linalg.norm(want / 2.0 ** 110)
+    assert (got[:, 1 % N] == 0).all()
+    s[:] = 2.0 ** 20                               # and those that it does not hold are infinite
+    q[:, :] = 127
+    x[:] = 2.0 ** 118
+    assert np.isposinf(_run(gpu, x, q, s)).all()
