@@ -47,6 +47,9 @@ def _oracle(x, w, b, H, batch, causal):
     (2, 64, 512, 256, 4, True),      # two sequences
     (1, 96, 3072, 256, 2, True),     # head dim 128, 8 K splits
     (1, 80, 768, 768, 12, False),    # full attention
+    (1, 100, 768, 256, 8, True),     # head dim 32: 4 splits, keys split over the wavefronts
+    (1, 96, 3072, 128, 4, False),    # head dim 32, 8 splits
+    (4, 65, 448, 1024, 32, True),    # head dim 32, 2 splits, 64 queries a block
 ])
 def test_qkv_attention_matches_composed_and_oracle(gpu, batch, T, K, d, H, causal):
     x, w, b = f32(batch * T, K), f32(K, 3 * d, scale=0.05), f32(3 * d, scale=0.1)
