@@ -343,7 +343,13 @@ void h16_tile_launch(int tile, const GArgs& p, hipStream_t s) {
 
 // Products with enough 128 x 64 tiles: fewer are left to gemm_mf, whose 64 x 64
 // tiles fill the chip or split K (777 x 1280 x 1280, 140 tiles: 17.8 us here,
-// 16.9 there; 200 x 248 x 4696, 148 tiles: 7.7 here, 10.9 there).
+// 16.9 there; 200 x 248 x 4696, 148 tiles: 7.7 here, 10.9 there).  Where it
+// splits K (few rows: fewer than a 64 x 64 tile a CU) it reads twice as fast, but
+// pays for the partial sums of every output: it wins from a k that grows with
+// their number (us here / there, weights not in cache; M x N x K: 64 x 10240 x 1280
+// 19.4 / 17.9, x 8192 99 / 51; 17 x 8192 x 768 12.4 / 9.5; 17 x 10240 x 8192 100 /
+// 45; 192 x 5120 x 1280 19 / 21, x 3072 40 / 25; with the weights in cache the two
+// meet at half as many k more).
 bool gemm_h16_ok(const Gemm& g, int cus) {
   const bool is16 = g.dt == DType::F16 || g.dt == DType::BF16;
   if (!(is16 && g.b_dt == g.dt && g.batch == 1 && !g.b_scale && !g.b_x3 && !g.a_x3 && !g.b_packed && !g.ln_gamma &&
@@ -352,6 +358,8 @@ bool gemm_h16_ok(const Gemm& g, int cus) {
     return false;
   // a tile's rows lie within the 2 GiB that a buffer resource spans
   if (g.a_sm < g.K || g.b_sn < g.K || g.a_sm >= (1 << 21) || g.b_sn >= (1 << 21)) return false;
+  const bool mf_splits = (g.M + 63) / 64 * ((g.N + 63) / 64) < cus;
+  if (mf_splits && g.K > 600 + g.M * g.N / 1000) return false;
   const int64_t tiles = h16_tiles(g, kH16Tiles[2]);
   return tiles >= (g.K <= 1024 ? cus / 2 : cus * 5 / 8) && tiles < (1LL << 31);
 }

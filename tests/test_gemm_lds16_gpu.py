@@ -95,6 +95,16 @@ def test_columns_of_a_tensor_past_2_gib(gpu, both):
     _close((xv @ gpu.transpose(wv)).to_numpy(), xs[:, :K] @ ws.T, "float16")
 
 
+@pytest.mark.parametrize("dt", ["float16", "bfloat16"])
+@pytest.mark.parametrize("M,N,K,here", [(17, 8192, 512, True), (64, 10240, 1024, True), (192, 5120, 1280, True),
+                                        (17, 8192, 768, False), (64, 10240, 1280, False), (17, 10240, 2048, False),
+                                        (192, 5120, 2048, False), (64, 16384, 2048, True)])
+def test_few_rows_of_long_k_are_left_to_split_tiles(gpu, M, N, K, here, dt):
+    assert _plan(M, N, K, dt).startswith("lds16" if here else "mf")
+    (x, xs), (w, ws), (b, bs) = (_dev(gpu, RNG.standard_normal(s) * 0.1, dt) for s in ((M, K), (N, K), (N,)))
+    _close(gpu.linear(x, w, b).to_numpy(), xs @ ws.T + bs, dt)
+
+
 def test_declines():
     assert not _plan(1024, 1280, 100).startswith("lds16")    # rows of partial vectors
     assert not _plan(100, 1280, 1280).startswith("lds16")    # too few tiles
