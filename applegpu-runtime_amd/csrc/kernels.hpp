@@ -429,6 +429,8 @@ struct AttnBwd {
   float scale = 1.f;
 };
 bool attention_backward_ok(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t D);
+// Whether it is faster there than the products over [Tq, Tk] one by one.
+bool attention_backward_pays(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t D, bool causal);
 bool attention_backward_rows_ok(const void* p, int64_t sb, int64_t sh, int64_t st);
 void attention_backward(const AttnBwd& a, hipStream_t s);
 // Whether attention can read Q/K/V as projection partials (fp32 MFMA kernel:

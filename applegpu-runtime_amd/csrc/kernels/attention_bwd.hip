@@ -40,6 +40,8 @@
 #include "device.hpp"
 #include "gemm_kernels.hpp"  // split_bf16x2
 
+#include <algorithm>
+#include <array>
 #include <type_traits>
 
 namespace agpu {
@@ -427,6 +429,37 @@ bool attention_backward_ok(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t
   const int64_t tiles = (Tq + 31) / 32 + (Tk + 31) / 32;
   return (D == 32 || D == 64 || D == 128) && Tq > 0 && Tk > 0 && B > 0 && H > 0 && Tq < (1 << 28) && Tk < (1 << 28) &&
          B * H < (1 << 28) && B * H * tiles < 0x7fffffffLL;
+}
+
+// A block walks the other side's rows one tile after the other, so with few
+// heads and a long side most CUs idle for the whole walk, where the
+// composition's products spread over the chip.  Both times, in us, from what
+// was measured at 1 to 48 heads, 16 to 4096 rows a side, MI355X (fused /
+// composed; not causal):
+//   heads x Tq x Tk   1 x 2048 x 2048   16 x 1024 x 1024   1 x 16 x 2048
+//   D = 32            93 / 130          67 / 251           79 / 91
+//   D = 64            168 / 139         107 / 267          117 / 90
+//   D = 128           214 / 151         297 / 329          164 / 71
+// The walk's time a 64-row tile (statistics; dQ; dK and dV) or, with more
+// blocks than CUs, the blocks' shares of it.  The composition: its launches
+// and its passes over [Tq, Tk], half as fast where rows of Tk floats are not
+// 16-byte aligned.  Of 954 measured shapes the fused kernels lost more than 5%
+// at 150 (3.8 times at worst), the choice by these times at 18 (1.4 times).
+bool attention_backward_pays(int64_t B, int64_t H, int64_t Tq, int64_t Tk, int64_t D, bool causal) {
+  constexpr float kCus = 256.f;
+  const int i = D == 32 ? 0 : D == 64 ? 1 : 2;
+  const float t_stats = std::array{0.95f, 1.45f, 2.2f}[i], t_q = std::array{1.35f, 2.1f, 2.9f}[i];
+  const float t_kv = std::array{1.9f, 3.6f, 4.4f}[i], t_elem = std::array{12.f, 12.5f, 15.f}[i] * 1e-6f;
+  const int64_t own = D == 128 ? 32 : 64;
+  const float bh = (float)(B * H), q_blocks = bh * (float)((Tq + own - 1) / own);
+  const float kv_blocks = bh * (float)((Tk + own - 1) / own);
+  const float q_walk = (float)(((causal ? std::min(Tq, Tk) : Tk) + 63) / 64), kv_walk = (float)((Tq + 63) / 64);
+  const float seen = causal ? 0.5f : 1.f;
+  const float stats = q_walk * t_stats * std::max(1.f, seen * q_blocks / kCus);
+  const float grads = std::max({kv_walk * t_kv, q_walk * t_q,
+                                seen * (kv_blocks * kv_walk * t_kv + q_blocks * q_walk * t_q) / kCus});
+  const float composed = 85.f + t_elem * (Tk % 4 != 0 ? 2.f : 1.f) * bh * (float)Tq * (float)Tk;
+  return 12.f + stats + grads <= composed;
 }
 
 void attention_backward(const AttnBwd& a, hipStream_t s) {

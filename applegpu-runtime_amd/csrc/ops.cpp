@@ -1641,8 +1641,8 @@ TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool ca
 }
 
 // (dq, dk, dv) of attention(q, k, v) for the output's gradient; one that is
-// not needed comes back null.  fp32 heads that attention_bwd.hip takes run
-// there, unless the native fp32 products are chosen (it multiplies split
+// not needed comes back null.  fp32 heads that attention_bwd.hip takes and
+// is faster for run there, unless the native fp32 products are chosen (it multiplies split
 // operands, as the default GEMMs do); others form P = softmax(q k^T s) (top-left causal mask, as torch's
 // is_causal), dV = P^T dO, dS = softmax_backward(dO V^T, P), dQ = s dS K and
 // dK = s dS^T Q on the GEMMs.
@@ -1658,7 +1658,8 @@ std::vector<TensorP> attention_backward(const TensorP& go, const TensorP& q, con
     a.B = nd == 4 ? q->shape[0] : 1;
     a.H = nd == 4 ? q->shape[1] : nd == 3 ? q->shape[0] : 1;
     a.Tq = q->shape[nd - 2]; a.Tk = kk->shape[nd - 2]; a.D = q->shape[nd - 1];
-    fused = k::attention_backward_ok(a.B, a.H, a.Tq, a.Tk, a.D);
+    fused = k::attention_backward_ok(a.B, a.H, a.Tq, a.Tk, a.D) &&
+            k::attention_backward_pays(a.B, a.H, a.Tq, a.Tk, a.D, causal);
   }
   if (!fused) {
     TensorP p = softmax(unary(k::kScale, matmul(q, kk, false, true), scale), causal ? k::kSoftmaxCausal : k::kSoftmax);

@@ -127,3 +127,23 @@ def test_native_fp32_products(torch_dev):
         _check(torch, got, _reference(torch, q, k, v, go, True), bar=1e-6)
     finally:
         lib.applegpu_ffi_gemm_tune(0, -1, 0)
+
+
+@pytest.mark.parametrize("H,Tq,Tk,D,causal,fused", [
+    (12, 128, 128, 64, True, True), (1, 16, 2048, 64, False, False), (1, 16, 2048, 64, True, True),
+    (2, 2048, 16, 128, False, False), (1, 2048, 2048, 128, True, False), (12, 1024, 1024, 128, True, True),
+    (1, 1023, 2049, 64, False, True), (3, 130, 4096, 32, False, False)])
+def test_the_faster_way_is_taken(torch_dev, gpu, H, Tq, Tk, D, causal, fused):
+    """A few heads with one long side take the products one by one: each of
+    the fused kernels' blocks would walk that side alone."""
+    torch = torch_dev
+    torch.manual_seed(12)
+    q, go = torch.randn(1, H, Tq, D), torch.randn(1, H, Tq, D)
+    k, v = torch.randn(1, H, Tk, D), torch.randn(1, H, Tk, D)
+    dev = [t.to("applegpu").requires_grad_(True) for t in (q, k, v)]
+    out = torch.nn.functional.scaled_dot_product_attention(*dev, is_causal=causal)
+    god = go.to("applegpu")
+    before = gpu.graph_stats()["launcher_calls"]
+    got = torch.autograd.grad(out, dev, god)
+    assert (gpu.graph_stats()["launcher_calls"] - before <= 2) == fused
+    _check(torch, (out,) + got, _reference(torch, q, k, v, go, causal))
