@@ -596,6 +596,11 @@ int32_t applegpu_ffi_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, i
     if (!out || cap == 0) fail("gemm_plan: null output buffer");
     k::Gemm g;
     g.dt = g.b_dt = wire(dtype_i8);
+    const float scale = 1.f;
+    if (g.dt == DType::I8) {  // linear_int8: fp32 rows, int8 codes with scales
+      g.dt = DType::F32;
+      g.b_scale = &scale;
+    }
     g.M = M; g.N = N; g.K = K; g.batch = batch;
     g.a_sk = a_kcontig ? 1 : M; g.a_sm = a_kcontig ? K : 1;
     g.b_sk = b_kcontig ? 1 : N; g.b_sn = b_kcontig ? K : 1;

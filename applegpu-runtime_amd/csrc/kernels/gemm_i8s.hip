@@ -269,12 +269,15 @@ int i8s_strips(const Gemm& g) { return g.M <= 32 ? 1 : 2; }
 
 }  // namespace
 
-// Ranges of K, by time: a phase takes a block about 2.3 us at one row strip
-// (8192 x 8192 codes, one row: 19 us) and 3.2 us at two (64 rows: 26 us), and
+// Ranges of K, by time: 2.3 us a phase at one row strip and 3.2 at two, a
+// launch's start and end spread over the 8 phases that a block of 8192 x 8192
+// codes has in it (at more phases each takes 1.5 and 1.9 us), and
 // each range writes and the reduction reads M x N floats, about 4 bytes a ps
 // for the whole chip, after a launch of 3 us and 0.25 us for each range that
 // an output's thread adds (64 x 8192 x 512: 17 us in 32 ranges, 35 in 64).
-// Grids stay within one block per CU.
+// Grids stay within one block per CU.  Over 1 to 128 rows of 256 x 512 to 8192
+// x 8192 codes the choice is within 2% of the best power of two, 18% at worst
+// (32 x 8192 x 512: 11.4 us in 4 ranges, 9.7 in one).
 int gemm_i8_stream_splits(const Gemm& g, int cus) {
   const int64_t rows = 32 * i8s_strips(g);
   const int64_t blocks = (g.N + kI8Cols - 1) / kI8Cols * ((g.M + rows - 1) / rows);
@@ -295,17 +298,40 @@ int gemm_i8_stream_splits(const Gemm& g, int cus) {
   return best;
 }
 
-// Up to 64 rows always (us, tiles -> this, codes not in cache): 1 x 8192 x 8192
-// 57 -> 24, 64 x 8192 x 8192 53 -> 35, 8 x 4096 x 4096 20 -> 13, 1 x 256 x 256
-// 7.9 -> 6.7.  More rows read the codes once per 64 and still gain where the
-// codes are many (128 x 8192 x 8192 127 -> 55, 256 x 8192 x 8192 178 -> 89, 100 x
-// 2048 x 2048 18.1 -> 17.7) or the tiles load them masked (K no multiple of 16:
-// 200 x 5000 x 300 43 -> 19, 256 x 300 x 300 20 -> 13); in between the tiles keep
-// their larger grids (128 x 768 x 3072 14.6, here 16.5).
+// Where the codes are streamed, over rows x columns x k (us, tiles -> this, codes
+// not in cache).  A launch here starts with two phases of loads and ends with a
+// reduction; the tiles start faster and have larger grids, so below some k they
+// win, the sooner the more rows there are:
+//  - to 16 rows from 128 k (16 x 1024 x 64: 5.6 -> 9.1, x 128: equal, 1 x 8192 x
+//    8192: 50 -> 23, 8 x 4096 x 4096: 20 -> 13), to 32 rows from 256 k (32 x 1024
+//    x 128: 1.1 times as long here, x 512: 0.88);
+//  - to 64 rows, two row strips a block, from 4096 k, or 3072 of as many columns
+//    (64 x 8192 x 512: 1.4 times as long here, x 2048: 1.1, x 3072: 0.89, x 8192:
+//    55 -> 35; 64 x 1024 x 4096: 1.0);
+//  - more rows read the codes once per 64 and gain where the codes are many: to
+//    128 rows from 6 M codes (100 x 2048 x 2048: 1.0, 128 x 4096 x 2048: 0.97, 128
+//    x 8192 x 8192: 0.39), to 256 from 4 M, where the tiles' grid leaves a short
+//    last round (256 x 4096 x 2048: 0.79, 256 x 8192 x 768: 0.88, 256 x 4096 x
+//    1024: 1.2, so the shorter k only with many columns), each from 2048 k, or
+//    with 8192 k whatever the columns (100 x 256 x 8192: 0.75);
+//  - rows that 16 bytes do not divide, which the tiles load masked: from 128 k, to
+//    256 rows from 192 (64 x 256 x 100: 1.6, 256 x 300 x 300: 20 -> 13, 200 x 8192
+//    x 8191: 0.24).
+static bool i8_stream_pays(int64_t M, int64_t N, int64_t K) {
+  constexpr int64_t kM = 1 << 20;
+  if (M <= 16) return K >= 128;
+  if (K % 16 != 0) return K >= (M <= 32 ? 128 : 192);
+  if (M <= 32) return K >= 256;
+  if (M <= 64) return K >= 4096 || (K >= 3072 && N >= 3072);
+  if (K >= 8192) return true;
+  if (M <= 128) return K >= 2048 && N * K >= 6 * kM;
+  return N * K >= 4 * kM && (K >= 2048 || N >= 6144);
+}
+
 bool gemm_i8_stream_ok(const Gemm& g) {
   return g.dt == DType::F32 && g.b_dt == DType::I8 && g.b_scale && g.batch == 1 && g.a_sk == 1 && g.b_sk == 1 &&
          g.M >= 1 && g.M <= 256 && g.N >= 1 && g.K >= 16 && g.K < (1LL << 30) &&
-         (g.M <= 64 || g.K % 16 != 0 || g.N * g.K >= (4LL << 20)) && g.alpha == 1.f && !g.bias && !g.residual &&
+         i8_stream_pays(g.M, g.N, g.K) && g.alpha == 1.f && !g.bias && !g.residual &&
          !g.mask && g.act == 0 && !g.b_x3 && !g.a_x3 && !g.b_packed && !g.ln_gamma && !g.c_pk && !g.pln_y && !g.pln_ypk &&
          !g.no_reduce && !g.a_rowsum_acc && !g.rs_out && !g.rs_in && (g.N + kI8Cols - 1) / kI8Cols <= 0x1000000;
 }

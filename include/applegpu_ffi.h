@@ -284,7 +284,8 @@ int32_t applegpu_ffi_x3_rows_out(int64_t M, int64_t N, int64_t K);
 int32_t applegpu_ffi_eval_many(const uint64_t* tensor_ids, uint32_t n);
 /* The plan the GEMM heuristic picks for an M x N x K (batch) problem of the
  * given dtype and operand layouts (a_kcontig: A(m,k) has unit k stride;
- * b_kcontig: B(k,n) has unit k stride), written as text into out. */
+ * b_kcontig: B(k,n) has unit k stride), written as text into out.  int8 means
+ * linear_int8's product: fp32 A, int8 B with a scale per column. */
 int32_t applegpu_ffi_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t batch, int8_t dtype_i8,
                                bool a_kcontig, bool b_kcontig, char* out, uint32_t cap);
 
