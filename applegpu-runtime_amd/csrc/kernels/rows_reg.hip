@@ -240,9 +240,13 @@ __global__ void __launch_bounds__(W == 1 ? 256 : 64 * W) layer_norm_reg(const T*
 }
 
 // How many wavefronts own a row (W) and how many vectors a thread holds (NV),
-// by the row's bytes: one wavefront up to 8 KB, so that short rows need no
-// barrier and fill the chip; 16 wavefronts beyond 32 KB keep a thread's share
-// within the 128 registers that a 1024-thread block leaves it.
+// by the row's bytes: one wavefront up to 4 KB, so that short rows need no
+// barrier and fill the chip; four to 32 KB (one with 8 vectors a lane took longer
+// from 4 to 8 KB: layer_norm of fp16 16 x 2049 7.4 -> 4.6 us, 2048 x 3000 10.9 ->
+// 9.4, softmax 300 x 4096 5.4 -> 4.3; of 8192 rows most gain, fp32 8192 x 1025
+// loses, 16.7 -> 18.8); 16
+// beyond, which keeps a thread's share within the 128 registers that a
+// 1024-thread block leaves it.
 constexpr int64_t kRegRowMax32 = 212992;  // fp32: 13 vectors of 16 wavefronts
 constexpr int64_t kRegRowMax16 = 131072;  // 16-bit: 8
 
@@ -253,7 +257,7 @@ void by_row_bytes(int64_t bytes, F f) {
   if (bytes <= 1024) AGPU_ROW(1, 1);
   else if (bytes <= 2048) AGPU_ROW(1, 2);
   else if (bytes <= 4096) AGPU_ROW(1, 4);
-  else if (bytes <= 8192) AGPU_ROW(1, 8);
+  else if (bytes <= 8192) AGPU_ROW(4, 2);
   else if (bytes <= 16384) AGPU_ROW(4, 4);
   else if (bytes <= 32768) AGPU_ROW(4, 8);
   else if (bytes <= 65536) AGPU_ROW(16, 4);

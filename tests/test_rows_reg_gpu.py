@@ -2,8 +2,8 @@
 rows (16-byte vectors in registers) against float64.
 
 Sizes: both sides of every change of wavefronts and vectors per thread, the
-last size the registers hold and the first past it, rows that end inside a
-vector, and fewer rows than a block takes.  Bars: fp32 sums of at most 52
+last size the registers hold and the first past it (of fp32 and of the 16-bit
+types), rows that end inside a vector, and fewer rows than a block takes.  Bars: fp32 sums of at most 52
 terms a thread, then a tree: 64 * 2^-24 = 4e-6 relative, log_softmax the same
 absolute per unit of its magnitude; 16-bit results are one rounding of the
 result (2^-11, 2^-8) plus the fp32 error."""
@@ -12,7 +12,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-COLS = [257, 300, 511, 513, 1023, 1025, 2047, 2049, 4096, 4099, 8192, 8193, 16385, 32769, 50257, 53248, 53249]
+COLS = [257, 300, 511, 513, 1023, 1025, 2047, 2049, 4096, 4099, 8192, 8193, 16385, 32769, 50257, 53248, 53249, 65536, 65537]
 BAR = {"float32": 4e-6, "float16": 2.0 ** -11 + 4e-6, "bfloat16": 2.0 ** -8 + 4e-6}
 
 
