@@ -375,13 +375,9 @@ void gemm_h16(const Gemm& g, const GArgs& p_in, int cus, hipStream_t s) {
   check_launch("gemm_h16");
 }
 
-// "h16 256x256" is a single round of whole stages, "lds16" any other grid.
 const char* gemm_h16_name(const Gemm& g, int cus) {
   static const char* names[3] = {"lds16 256x256", "lds16 128x128", "lds16 128x64"};
-  const int tile = h16_pick(g, cus);
-  const int64_t tiles = h16_tiles(g, kH16Tiles[tile]);
-  if (tile == 0 && g.K % 64 == 0 && tiles * 4 >= (int64_t)cus * 3 && tiles <= cus) return "h16 256x256";
-  return names[tile];
+  return names[h16_pick(g, cus)];
 }
 
 }  // namespace k
