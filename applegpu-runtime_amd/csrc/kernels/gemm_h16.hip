@@ -5,8 +5,8 @@
 // crates/core/src/kernel_templates.rs:987-1072).
 //
 // One block owns a BM x BN tile over the whole K, in stages of 64 k:
-//  - Global -> LDS with global_load_lds_dwordx4: each wave instruction
-//    copies one 1 KB window of 8 rows x 64 k into LDS with no register
+//  - Global -> LDS with buffer loads to LDS of 16 bytes a lane: each wave
+//    instruction copies one 1 KB window of 8 rows x 64 k with no register
 //    staging.  Lane p of the instruction reads row p / 8 of the window, whose
 //    128 bytes are one contiguous read; the row's 16-byte chunks land
 //    exchanged (chunk ^ (row / 2) % 8), so that the 16 lanes of a fragment
@@ -23,8 +23,6 @@
 //    bytes a lane, whole 128-byte runs of a row, at any alignment (the
 //    50257-column head's rows start at odd addresses).
 #include "gemm_kernels.hpp"
-
-#include <type_traits>
 
 namespace agpu {
 namespace k {
@@ -74,16 +72,17 @@ __device__ __forceinline__ float h16_act(float v) {
   else return v;
 }
 
-template <typename T, int TM, int TN, int WM, int WN, int BK, int NB, int ACT>
+template <typename T, int TM, int TN, int WM, int WN, int ACT>
 __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) gemm_h16_kernel(GArgs p) {
   constexpr int NW = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
+  constexpr int BK = 64;                                  // k per stage
   constexpr int CH = BK / 8, WR = 64 / CH, KK = BK / 16;  // chunks per row, rows per 1 KB window, MFMA steps per stage
   constexpr int AW = BM / WR, BW = BN / WR;               // windows per stage
   constexpr int STAGE = (AW + BW) * 512;   // elements
   constexpr int LA = AW / NW, LB = BW / NW, LPW = LA + LB;  // window copies per wavefront per stage
   static_assert(AW % NW == 0 && BW % NW == 0, "tile shape");
   typedef typename Mfma32h<T>::vec V8;
-  __shared__ __attribute__((aligned(16))) T lds[NB * STAGE];
+  __shared__ __attribute__((aligned(16))) T lds[2 * STAGE];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int tmi, tni;
   tile_coords(p, tmi, tni);
@@ -106,8 +105,8 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
     off[q] = (int)((r * (q < LA ? p.a_sm : p.b_sn) + ((lane % CH) ^ swz(r)) * 8) * (int64_t)sizeof(T));
   }
   auto issue = [&](int st) __attribute__((always_inline)) {
-    T* da = lds + (st % NB) * STAGE + w * LA * 512;
-    T* db = lds + (st % NB) * STAGE + (AW + w * LB) * 512;
+    T* da = lds + (st % 2) * STAGE + w * LA * 512;
+    T* db = lds + (st % 2) * STAGE + (AW + w * LB) * 512;
     const int k = st * (BK * (int)sizeof(T));
     const bool ends = (st + 1) * BK > (int)p.K;
     if (ends) {
@@ -133,7 +132,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
   auto foff = [&](int r, int c) { return r * BK + ((c ^ swz(r)) * 8); };
   V8 fa[2][TM], fb[2][TN];
   auto read = [&](int set, int st, int kk) __attribute__((always_inline)) {
-    const T* a = lds + (st % NB) * STAGE;
+    const T* a = lds + (st % 2) * STAGE;
     const T* b = a + AW * 512;
 #pragma unroll
     for (int j = 0; j < TN; ++j) fb[set][j] = *(const V8*)(b + foff((wn * TN + j) * 32 + l31, 2 * kk + hi));
@@ -154,21 +153,11 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
       for (int j = 0; j < TN; ++j) acc[i][j] = Mfma32h<T>::run(fb[set][j], fa[set][i], acc[i][j]);
   };
 
-  // waits until at most n of this wavefront's copies are in flight, and with
-  // DS for its LDS reads
-  auto wait = [&](auto n, auto ds) __attribute__((always_inline)) {
-    constexpr int v = decltype(n)::value;
-    __builtin_amdgcn_s_waitcnt((v & 15) | ((v >> 4) << 14) | (decltype(ds)::value ? 0x0070 : 0x0f70));
-  };
-  typedef std::integral_constant<int, (NB - 2) * LPW> Ahead;
-  typedef std::integral_constant<int, 0> None;
-#pragma unroll
-  for (int st = 0; st < NB - 1; ++st)
-    if (st < nk) issue(st);
-  if (nk >= NB - 1) wait(Ahead{}, std::false_type{});
-  else wait(None{}, std::false_type{});
+  constexpr int kCopies = 0x0f70, kCopiesAndReads = 0x0070;  // waits for this wavefront's copies, and its LDS reads
+  issue(0);
+  __builtin_amdgcn_s_waitcnt(kCopies);
   __syncthreads();
-  if (NB - 1 < nk) issue(NB - 1);
+  if (nk > 1) issue(1);
   read(0, 0, 0);
   for (int st = 0; st < nk; ++st) {
     // the fragments read before the last MFMAs are there by now; without this
@@ -185,11 +174,10 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
     }
     // this wavefront holds the rest of stage st in registers, and its copies
     // of stage st + 1 have landed; after the barrier so for every wavefront
-    if (st + NB <= nk) wait(Ahead{}, std::true_type{});
-    else wait(None{}, std::true_type{});
+    __builtin_amdgcn_s_waitcnt(kCopiesAndReads);
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    if (st + NB < nk) issue(st + NB);
+    if (st + 2 < nk) issue(st + 2);
     if (st + 1 < nk) read(0, st + 1, 0);
     __builtin_amdgcn_sched_barrier(0);
     mul((KK - 1) & 1);
@@ -201,7 +189,7 @@ __global__ void __launch_bounds__(64 * WM * WN, WM * WN <= 4 ? 1 : WM * WN / 4) 
   // of LDS, 32 rows x 32 TN columns of fp32 at a time, rows 4 floats apart.
   constexpr int CN = 32 * TN, CP = CN + 4;
   constexpr int LPR = CN / 8, RPI = 64 / LPR;  // lanes per row, rows per instruction
-  static_assert(NW * 32 * CP * 4 <= NB * STAGE * (int)sizeof(T), "epilogue staging");
+  static_assert(NW * 32 * CP * 4 <= 2 * STAGE * (int)sizeof(T), "epilogue staging");
   float* ct = (float*)lds + w * 32 * CP;
   const T* bias = (const T*)p.bias;
   const T* R = (const T*)p.res;
@@ -322,7 +310,7 @@ int h16_pick(const Gemm& g, int cus) {
 template <typename T, int TM, int TN, int WM, int WN>
 void h16_launch(const GArgs& p, hipStream_t s) {
   const dim3 grid((unsigned)(p.tiles_m * p.tiles_n)), block(64 * WM * WN);
-#define AGPU_H16(ACT) hipLaunchKernelGGL((gemm_h16_kernel<T, TM, TN, WM, WN, 64, 2, ACT>), grid, block, 0, s, p)
+#define AGPU_H16(ACT) hipLaunchKernelGGL((gemm_h16_kernel<T, TM, TN, WM, WN, ACT>), grid, block, 0, s, p)
   switch (p.act) {
     case kActNone: AGPU_H16(kActNone); break;
     case kActRelu: AGPU_H16(kActRelu); break;
