@@ -991,7 +991,7 @@ unsigned rows_grid(int64_t rows) { return (unsigned)((rows + kRowsPerBlock - 1) 
 // and the packed outputs build on them), and those under 256 columns, where
 // rows_reg.hip's 16-byte vectors leave lanes idle (fp16 8192 x 64: softmax
 // 4.4 us here, 5.3 there).  The others are faster there: softmax 4096 x 777
-// 11.4 -> 8.0 us in fp32 and 12.5 -> 6.4 us in fp16, 2047 x 50257 fp32
+// 11.4 -> 8.0 us in fp32 and 12.5 -> 6.6 us in fp16, 2047 x 50257 fp32
 // 340 -> 182 us (4.5 TB/s), layer_norm 512 x 16000 fp32 67 -> 15 us.
 bool wave_row_ok(int64_t cols, bool vec) { return cols < 256 || (vec && cols <= 2048 && cols % 256 == 0); }
 
