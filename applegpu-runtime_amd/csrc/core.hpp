@@ -205,6 +205,9 @@ class Runtime {
 
   // Resource limits (crates/core/src/limits.rs:39-77); 0 = unlimited.
   size_t max_tensor_bytes = 0, max_memory_bytes = 0, max_tensors = 0;
+  // Whether they leave room for tensors of `total` bytes, the largest of
+  // `largest`.
+  bool fits(size_t largest, size_t total) const;
 
   // Optional host-visible allocations (APPLEGPU_HOST_VISIBLE=1) for callers
   // that poke returned pointers from the host.

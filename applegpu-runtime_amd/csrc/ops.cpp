@@ -1641,25 +1641,36 @@ TensorP attention(const TensorP& q, const TensorP& kk, const TensorP& v, bool ca
 }
 
 // (dq, dk, dv) of attention(q, k, v) for the output's gradient; one that is
-// not needed comes back null.  fp32 heads that attention_bwd.hip takes and
-// is faster for run there, unless the native fp32 products are chosen (it multiplies split
-// operands, as the default GEMMs do); others form P = softmax(q k^T s) (top-left causal mask, as torch's
-// is_causal), dV = P^T dO, dS = softmax_backward(dO V^T, P), dQ = s dS K and
-// dK = s dS^T Q on the GEMMs.
+// not needed comes back null.  fp32 heads that attention_bwd.hip takes and is
+// faster for run there, unless the native fp32 products are chosen (it
+// multiplies split operands, as the default GEMMs do); others form P =
+// softmax(q k^T s) (top-left causal mask, as torch's is_causal), dV = P^T dO,
+// dS = softmax_backward(dO V^T, P), dQ = s dS K and dK = s dS^T Q on the
+// GEMMs.  Of two ways that could run, one that a memory limit would refuse
+// gives way to the other.
 std::vector<TensorP> attention_backward(const TensorP& go, const TensorP& q, const TensorP& kk, const TensorP& v,
                                         bool causal, float scale, bool need_q, bool need_k, bool need_v) {
   const int nd = q->ndim;
   bool fused = q->dtype == DType::F32 && kk->dtype == DType::F32 && v->dtype == DType::F32 &&
-               go->dtype == DType::F32 && k::gemm_tune().f32_mode != k::kF32Native && nd >= 2 && nd <= 4 && kk->ndim == nd && v->dims() == kk->dims() &&
-               go->dims() == q->dims();
+               go->dtype == DType::F32 && k::gemm_tune().f32_mode != k::kF32Native && nd >= 2 && nd <= 4 &&
+               kk->ndim == nd && v->dims() == kk->dims() && go->dims() == q->dims();
   for (int i = 0; fused && i < nd; ++i) fused = i == nd - 2 || kk->shape[i] == q->shape[i];
   k::AttnBwd a;
   if (fused) {
     a.B = nd == 4 ? q->shape[0] : 1;
     a.H = nd == 4 ? q->shape[1] : nd == 3 ? q->shape[0] : 1;
     a.Tq = q->shape[nd - 2]; a.Tk = kk->shape[nd - 2]; a.D = q->shape[nd - 1];
-    fused = k::attention_backward_ok(a.B, a.H, a.Tq, a.Tk, a.D) &&
-            k::attention_backward_pays(a.B, a.H, a.Tq, a.Tk, a.D, causal);
+    fused = k::attention_backward_ok(a.B, a.H, a.Tq, a.Tk, a.D);
+  }
+  if (fused) {
+    const size_t scores = (size_t)(a.B * a.H * a.Tq) * a.Tk * sizeof(float), gq = need_q ? q->nbytes() : 0;
+    // three arrays of scores at a time and a product's partial sums; the fused kernel writes dk and dv together
+    const bool composed_fits =
+        rt().fits(scores, 4 * scores + gq + (need_k ? kk->nbytes() : 0) + (need_v ? v->nbytes() : 0));
+    const bool fused_fits =
+        rt().fits(std::max(gq, kk->nbytes()), gq + (need_k || need_v ? kk->nbytes() + v->nbytes() : 0));
+    fused = composed_fits && fused_fits ? k::attention_backward_pays(a.B, a.H, a.Tq, a.Tk, a.D, causal)
+                                        : !composed_fits;
   }
   if (!fused) {
     TensorP p = softmax(unary(k::kScale, matmul(q, kk, false, true), scale), causal ? k::kSoftmaxCausal : k::kSoftmax);

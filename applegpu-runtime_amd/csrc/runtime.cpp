@@ -439,6 +439,11 @@ Runtime& Runtime::get() {
   return *g_rt;
 }
 
+bool Runtime::fits(size_t largest, size_t total) const {
+  return (!max_tensor_bytes || largest <= max_tensor_bytes) &&
+         (!max_memory_bytes || pool_->stats().live_bytes + total <= max_memory_bytes);
+}
+
 TensorP Runtime::alloc(DType dt, const std::vector<int64_t>& dims) {
   TensorP t = make_meta(dt, dims);
   size_t nb = t->nbytes();

@@ -147,3 +147,26 @@ def test_the_faster_way_is_taken(torch_dev, gpu, H, Tq, Tk, D, causal, fused):
     got = torch.autograd.grad(out, dev, god)
     assert (gpu.graph_stats()["launcher_calls"] - before <= 2) == fused
     _check(torch, (out,) + got, _reference(torch, q, k, v, go, causal))
+
+
+def test_memory_limits_choose_the_way_that_fits(torch_dev, gpu):
+    """One head of 2048 x 2048 takes the products over [2048, 2048] by itself,
+    and the fused kernels where a limit leaves no room for those."""
+    torch = torch_dev
+    torch.manual_seed(13)
+    q, k, v, go = (torch.randn(1, 1, 2048, 128) for _ in range(4))
+    want = _reference(torch, q, k, v, go, False)
+    dev = [t.to("applegpu").requires_grad_(True) for t in (q, k, v)]
+    out = torch.nn.functional.scaled_dot_product_attention(*dev)
+    god = go.to("applegpu")
+    for limit, fused in ((dict(), False), (dict(max_tensor_size_mb=8), True),
+                         (dict(max_memory_mb=(gpu.memory_usage() >> 20) + 24), True)):
+        gpu.set_limits(**limit)
+        try:
+            before = gpu.graph_stats()["launcher_calls"]
+            got = torch.autograd.grad(out, dev, god, retain_graph=True)
+            assert (gpu.graph_stats()["launcher_calls"] - before <= 2) == fused
+        finally:
+            gpu.set_limits()
+        _check(torch, (out,) + got, want)
+        del got
